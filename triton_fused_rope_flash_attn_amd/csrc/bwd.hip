@@ -769,6 +769,9 @@ bwd_dkdv_kernel(const BwdParams p) {
   // 16-bit operands: Q-hat^T and dO^T are read transposed from sQ / sG
   // (ds_read_b64_tr_b16); fp32 storage keeps explicit transposed copies.
   constexpr bool TR = sizeof(S) == 2;
+  // two query blocks in flight per trip, where the registers allow it (at D 32
+  // it measured +11%: the second block's accumulators cost a wave per SIMD)
+  constexpr bool PIPE2 = sizeof(S) == 2 && (KT == 1 || D == 64);
 
   static_assert(!FS || CT == DT_BF16, "fp16 logit operands go with bf16 compute");
   __shared__ __attribute__((aligned(16))) S sQ[QS * LDQ];
@@ -1033,37 +1036,53 @@ bwd_dkdv_kernel(const BwdParams p) {
     lds_barrier();
     }
 
-    // S and dP of query block j for key subtile u.  -LSE2 and -delta of
+    // S and dP of query block j for the wave's key subtiles; each Q-hat / dO
+    // fragment is read once and feeds all KT of them.  (Read again per subtile,
+    // the LDS bound this kernel: D 64, N 4096, 48 planes, backward 804 -> 733
+    // us; fp32 compute, N 197, 16 planes 62 -> 55 us; bit-identical.)  -LSE2 and -delta of
     // queries 32j + 8lg + e, e = 4h + i, seed the accumulators of half h
     // (P = exp2(S), dP - delta need no arithmetic; queries >= N have
     // -LSE2 = -inf, so P = 0).
-    auto sp = [&](int j, int u, f32x4 (&sacc)[2], f32x4 (&pacc)[2]) __attribute__((always_inline)) {
-        sacc[0] = *reinterpret_cast<const f32x4*>(&sL2[32 * j + 8 * lg]);
-        sacc[1] = *reinterpret_cast<const f32x4*>(&sL2[32 * j + 8 * lg + 4]);
-        pacc[0] = *reinterpret_cast<const f32x4*>(&sDl[32 * j + 8 * lg]);
-        pacc[1] = *reinterpret_cast<const f32x4*>(&sDl[32 * j + 8 * lg + 4]);
+    using Acc = f32x4[KT][2];
+    auto sp = [&](int j, Acc& sacc, Acc& pacc) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
+      for (int h = 0; h < 2; ++h) {
+        const f32x4 nl2 = *reinterpret_cast<const f32x4*>(&sL2[32 * j + 8 * lg + 4 * h]);
+        const f32x4 ndl = *reinterpret_cast<const f32x4*>(&sDl[32 * j + 8 * lg + 4 * h]);
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int ql = 32 * j + qrow(8 * (lr >> 2) + 4 * h + (lr & 3));
-            LFrag a;
-            if constexpr (FS)
-              a = LC::lds(&sQf[ql * LDQ + 32 * s + 8 * lg]);
-            else
-              a = C::lds(&sQ[ql * LDQ + 32 * s + 8 * lg]);
-            const Frag b = C::lds(&sG[ql * LDQ + 32 * s + 8 * lg]);
-            sacc[h] = LC::mma(a, kf[u][s], sacc[h]);
-            pacc[h] = C::mma(b, vf[u][s], pacc[h]);
+        for (int u = 0; u < KT; ++u) {
+          sacc[u][h] = nl2;
+          pacc[u][h] = ndl;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int ql = 32 * j + qrow(8 * (lr >> 2) + 4 * h + (lr & 3));
+          LFrag a;
+          if constexpr (FS)
+            a = LC::lds(&sQf[ql * LDQ + 32 * s + 8 * lg]);
+          else
+            a = C::lds(&sQ[ql * LDQ + 32 * s + 8 * lg]);
+          const Frag b = C::lds(&sG[ql * LDQ + 32 * s + 8 * lg]);
+#pragma unroll
+          for (int u = 0; u < KT; ++u) {
+            sacc[u][h] = LC::mma(a, kf[u][s], sacc[u][h]);
+            pacc[u][h] = C::mma(b, vf[u][s], pacc[u][h]);
           }
         }
+      }
     };
     // P and dS of query block j from its S / dP, then dV += P dO and
-    // dK-hat += dS Q-hat for key subtile u.
-    auto pdk = [&](int j, int u, const f32x4 (&sacc)[2], const f32x4 (&pacc)[2]) __attribute__((always_inline)) {
-        // Keys >= N (lane key kv0 + lr) need no mask: their K-hat and V rows
-        // are zero, so P and dS there are finite and only reach the dK / dV
-        // rows of those keys, which are never stored.
+    // dK-hat += dS Q-hat; each dO^T / Q-hat^T fragment feeds all KT subtiles.
+    auto pdk = [&](int j, const Acc& sacc, const Acc& pacc) __attribute__((always_inline)) {
+      // Keys >= N (lane key kv0 + lr; a whole subtile past it included) need
+      // no mask: their K-hat and V rows are zero, and P and dS there only
+      // reach the dK / dV rows of those keys, which are never stored.
+      Frag pf[KT], dsf[KT], dsfl[KT];
+#pragma unroll
+      for (int u = 0; u < KT; ++u) {
         float pv[8], dsv[8];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -1071,57 +1090,56 @@ bwd_dkdv_kernel(const BwdParams p) {
           for (int i = 0; i < 4; ++i) {
             const int e = 4 * h + i;
             // FS: the seeds are -LSE2 * fq * fk, so this is exp2(S - LSE2)
-            const float pr = fast_exp2(FS ? sacc[h][i] * fsc : sacc[h][i]);
+            const float pr = fast_exp2(FS ? sacc[u][h][i] * fsc : sacc[u][h][i]);
             pv[e] = pr;
-            dsv[e] = pr * pacc[h][i];
+            dsv[e] = pr * pacc[u][h][i];
           }
-        const Frag pf = C::make(pv);
-        Frag dsf, dsfl;
+        pf[u] = C::make(pv);
         if constexpr (FS)
-          split_bf16x8(dsv, dsf.v, dsfl.v);
+          split_bf16x8(dsv, dsf[u].v, dsfl[u].v);
         else
-          dsf = C::make(dsv);
-#pragma unroll
-        for (int d = 0; d < DT; ++d) {
-          // A = dO^T / Q-hat^T rows 16d.., k-slot e <-> query 32j + 8lg + e (the P / dS order)
-          Frag ag, aq;
-          if constexpr (TR) {
-            const int o0 = (32 * j + qt0) * LDQ + 16 * d + 4 * (lr & 3);
-            const int o1 = (32 * j + qt1) * LDQ + 16 * d + 4 * (lr & 3);
-            ag = C::tr(&sG[o0], &sG[o1]);
-            aq = C::tr(&sQ[o0], &sQ[o1]);
-          } else {
-            ag = C::lds(&sGt[(16 * d + lr) * LDT + 32 * j + 8 * lg]);
-            aq = C::lds(&sQt[(16 * d + lr) * LDT + 32 * j + 8 * lg]);
-          }
-          dvacc[u][d] = C::mma(ag, pf, dvacc[u][d]);
-          if constexpr (FS) dkacc[u][d] = C::mma(aq, dsfl, dkacc[u][d]);
-          dkacc[u][d] = C::mma(aq, dsf, dkacc[u][d]);
-        }
-    };
-
-    if constexpr (KT == 1 && sizeof(S) == 2) {
-      // Two query blocks per trip: the S / dP products of block j+1 go to the
-      // MFMA pipe before block j's probabilities are computed on the VALU (a
-      // ragged last block recomputes block j instead and skips its update).
-      if (kv_first < N) {   // wave-uniform
-        const int nbj = rows / 32;
-        for (int j = 0; j < nbj; j += 2) {
-          f32x4 sA[2], pA[2], sB[2], pB[2];
-          sp(j, 0, sA, pA);
-          sp(min(j + 1, nbj - 1), 0, sB, pB);
-          pdk(j, 0, sA, pA);
-          if (j + 1 < nbj) pdk(j + 1, 0, sB, pB);
-        }
+          dsf[u] = C::make(dsv);
       }
-    } else {
-      for (int j = 0; j < rows / 32; ++j) {
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        // A = dO^T / Q-hat^T rows 16d.., k-slot e <-> query 32j + 8lg + e (the P / dS order)
+        Frag ag, aq;
+        if constexpr (TR) {
+          const int o0 = (32 * j + qt0) * LDQ + 16 * d + 4 * (lr & 3);
+          const int o1 = (32 * j + qt1) * LDQ + 16 * d + 4 * (lr & 3);
+          ag = C::tr(&sG[o0], &sG[o1]);
+          aq = C::tr(&sQ[o0], &sQ[o1]);
+        } else {
+          ag = C::lds(&sGt[(16 * d + lr) * LDT + 32 * j + 8 * lg]);
+          aq = C::lds(&sQt[(16 * d + lr) * LDT + 32 * j + 8 * lg]);
+        }
 #pragma unroll
         for (int u = 0; u < KT; ++u) {
-          if (kv_first + 16 * u >= N) continue;   // wave-uniform
-          f32x4 sacc[2], pacc[2];
-          sp(j, u, sacc, pacc);
-          pdk(j, u, sacc, pacc);
+          dvacc[u][d] = C::mma(ag, pf[u], dvacc[u][d]);
+          if constexpr (FS) dkacc[u][d] = C::mma(aq, dsfl[u], dkacc[u][d]);
+          dkacc[u][d] = C::mma(aq, dsf[u], dkacc[u][d]);
+        }
+      }
+    };
+
+    if (kv_first < N) {   // wave-uniform
+      const int nbj = rows / 32;
+      if constexpr (PIPE2) {
+        // Two query blocks per trip: the S / dP products of block j+1 go to the
+        // MFMA pipe before block j's probabilities are computed on the VALU (a
+        // ragged last block recomputes block j instead and skips its update).
+        for (int j = 0; j < nbj; j += 2) {
+          Acc sA, pA, sB, pB;
+          sp(j, sA, pA);
+          sp(min(j + 1, nbj - 1), sB, pB);
+          pdk(j, sA, pA);
+          if (j + 1 < nbj) pdk(j + 1, sB, pB);
+        }
+      } else {
+        for (int j = 0; j < nbj; ++j) {
+          Acc sacc, pacc;
+          sp(j, sacc, pacc);
+          pdk(j, sacc, pacc);
         }
       }
     }
