@@ -129,7 +129,10 @@ size_t farope_attn_residual_elems(const farope_attn_desc* desc);
  * statistics; with a lone last key its dS per query row; one int32 exponent
  * per key tile; the key tiles' fp16 K-hat rows; and their fp16 dS^T rows
  * (pitch seq_len rounded up to 64), which the dQ GEMM reads instead of
- * recomputing the logits.  0 on an invalid descriptor.
+ * recomputing the logits.  At the streamed shapes (16-bit tensors computed in
+ * their own type, head_dim 64 and seq_len > 257 or head_dim 32 and seq_len >
+ * 256; each part from a 256-byte boundary): -delta and -LSE * log2(e) rows, then the rotated Q rows and the
+ * rotated, scaled K rows in 16 bits.  0 on an invalid descriptor.
  */
 size_t farope_attn_bwd_workspace_elems(const farope_attn_desc* desc);
 
@@ -146,6 +149,23 @@ int farope_attn_fwd(const farope_attn_desc* desc,
                     const float* rope_packed, size_t rope_elems,
                     void* o, const int64_t o_stride[4], void* o_res,
                     float* lse, void* stream);
+
+/*
+ * farope_attn_fwd with a caller workspace of farope_attn_fwd_workspace_elems(desc)
+ * fp32 elements (16-byte aligned; NULL: as farope_attn_fwd).  Where that is not
+ * 0 (16-bit tensors computed in their own type, head_dim 32 or 64, seq_len >
+ * 256) and every tensor allows vector access, the rotated K rows are written
+ * there once and streamed by every query tile; otherwise it is not used.  No
+ * counterpart in the reference.
+ */
+size_t farope_attn_fwd_workspace_elems(const farope_attn_desc* desc);
+int farope_attn_fwd_ws(const farope_attn_desc* desc,
+                       const void* q, const int64_t q_stride[4],
+                       const void* k, const int64_t k_stride[4],
+                       const void* v, const int64_t v_stride[4],
+                       const float* rope_packed, size_t rope_elems,
+                       void* o, const int64_t o_stride[4], void* o_res,
+                       float* lse, float* ws, void* stream);
 
 /* delta = rowsum(dout * (o + o_res)) in fp32 (o_res may be NULL).  Replaces
  * _attn_bwd_preprocess (launch FA:1076-1082; kernel FA:325-357). */
@@ -233,9 +253,10 @@ int farope_attn_bwd_noalloc(const farope_attn_desc* desc,
  * FA:76-90, FA:318-324, FA:359-373, FA:693-707).  which: 0 = forward,
  * 1 = backward.  out[0] = variant (fwd: 0 = persistent pipelined kernel,
  * 1 = one wave per (b, h) plane for 193 <= N <= 208 at head_dim 64 with
- * 16-bit tensors, assuming vector access; bwd: 0 fused, 1 split, 2 split with
+ * 16-bit tensors, assuming vector access (the streamed query tiles of
+ * farope_attn_fwd_ws are not reported); bwd: 0 fused, 1 split, 2 split with
  * the key-tile kernel, 3 key tiles that store dS and dQ as one GEMM over it,
- * assuming vector access), out[1] = query (fwd) or key (bwd) rows per work item,
+ * 4 streamed tiles, assuming vector access), out[1] = query (fwd) or key (bwd) rows per work item,
  * out[2] = work items per (b, h) plane, out[3] = threads per workgroup.  When 1 to 8 rows are left past out[1] * out[2] (N = 1025 with
  * 128- or 256-row items), they are computed by the tail-row kernels (or, for
  * a single row with fp16 logit operands, by one designated item of each plane

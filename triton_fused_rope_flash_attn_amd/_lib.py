@@ -33,6 +33,8 @@ EXPORTS = (
     "farope_attn_residual_elems",
     "farope_attn_bwd_workspace_elems",
     "farope_attn_fwd",
+    "farope_attn_fwd_workspace_elems",
+    "farope_attn_fwd_ws",
     "farope_attn_bwd_preprocess",
     "farope_attn_bwd_dk_dv",
     "farope_attn_bwd_dq",
@@ -72,6 +74,8 @@ _SIGNATURES = {
     "farope_attn_residual_elems": (ctypes.c_size_t, [_D]),
     "farope_attn_bwd_workspace_elems": (ctypes.c_size_t, [_D]),
     "farope_attn_fwd": (ctypes.c_int, [_D, _P, _S, _P, _S, _P, _S, _P, _Z, _P, _S, _P, _P, _P]),
+    "farope_attn_fwd_workspace_elems": (ctypes.c_size_t, [_D]),
+    "farope_attn_fwd_ws": (ctypes.c_int, [_D, _P, _S, _P, _S, _P, _S, _P, _Z, _P, _S, _P, _P, _P, _P]),
     "farope_attn_bwd_preprocess": (ctypes.c_int, [_D, _P, _S, _P, _P, _S, _P, _P]),
     "farope_attn_bwd_dk_dv": (
         ctypes.c_int,
@@ -167,11 +171,16 @@ def _ptr(t) -> int | None:
     return t.data_ptr() if t is not None and t.numel() > 0 else None
 
 
-def attn_fwd(desc: AttnDesc, q, k, v, rope, o, lse, o_res=None) -> None:
-    rc = load().farope_attn_fwd(
+def fwd_workspace_elems(desc: AttnDesc) -> int:
+    """fp32 elements of attn_fwd's workspace; see farope_attn_fwd_workspace_elems."""
+    return int(load().farope_attn_fwd_workspace_elems(ctypes.byref(desc)))
+
+
+def attn_fwd(desc: AttnDesc, q, k, v, rope, o, lse, o_res=None, ws=None) -> None:
+    rc = load().farope_attn_fwd_ws(
         ctypes.byref(desc),
         q.data_ptr(), strides(q), k.data_ptr(), strides(k), v.data_ptr(), strides(v),
-        rope.data_ptr(), rope.numel(), o.data_ptr(), strides(o), _ptr(o_res), lse.data_ptr(), stream_of(q),
+        rope.data_ptr(), rope.numel(), o.data_ptr(), strides(o), _ptr(o_res), lse.data_ptr(), _ptr(ws), stream_of(q),
     )
     check(rc, "farope_attn_fwd")
 

@@ -104,8 +104,11 @@ def attn_fwd(
     res = _uses_residual(io, compute_dtype, D)
     o_res = torch.empty((B, H, N, D) if res else (0,), dtype=q.dtype, device=q.device)
     desc = _lib.make_desc(B, H, N, D, n_pos, has_cls, io, compute_dtype, softmax_scale)
+    # rotated K rows of the streamed forward (none for the other kernels)
+    elems = _lib.fwd_workspace_elems(desc)
+    ws = torch.empty(elems, dtype=torch.float32, device=q.device) if elems else None
     with torch.cuda.device(q.device):
-        _lib.attn_fwd(desc, q, k, v, rope, o, lse, o_res)
+        _lib.attn_fwd(desc, q, k, v, rope, o, lse, o_res, ws)
     return o, lse, o_res
 
 

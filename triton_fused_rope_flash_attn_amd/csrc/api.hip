@@ -314,10 +314,48 @@ DsWs ds_ws(const farope_attn_desc* d) {
   return w;
 }
 
+// The streamed tiles (fwd_stream.hip, bwd_stream.hip): 16-bit tensors computed
+// in their own type at head_dim 32 or 64.  (Vector access to every tensor is
+// checked at the call.)
+bool stream_shape(const farope_attn_desc* d) {
+  if (d->io_dtype == FAROPE_F32 || d->io_dtype != d->compute_dtype) return false;
+  if (d->head_dim != 64 && d->head_dim != 32) return false;
+  return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kStreamTileRows) <= INT32_MAX;
+}
+// Forward: planes past the 256 rows whose table fwd_kernel keeps in LDS.
+// Measured (us, fwd_kernel / streamed, the K-hat pass included): D 64, N 577,
+// 384 planes 89 / 59; N 257, 1536 planes 90 / 78; N 256 52 / 59; N 170, 3072
+// planes 81 / 107.  D 32: N 257, 512 planes 32 / 25; N 256 15 / 20.
+bool fwd_stream(const farope_attn_desc* d) { return stream_shape(d) && d->seq_len > kPlaneMaxN; }
+// Backward: planes past the one-pass kernel's 256 rows at head_dim 64 (it
+// stays at N = 257, whose delta-only workspace callers rely on), and past the
+// same length at head_dim 32.  Measured (us, bwd_dq_kernel + bwd_dkdv_kernel /
+// streamed): D 64, N 577, 384 planes 264 / 165; N 4096, 48 planes 795 / 618;
+// N 324, 24 planes 42 / 24.  D 32, N 257, 512 planes 71 / 46.
+bool bwd_stream(const farope_attn_desc* d) {
+  return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim == 64 ? 1 : 0);
+}
+// Its workspace, in fp32 elements, each part from a 256-byte boundary:
+// -delta rows, -LSE2 rows, Q-hat rows and K-hat * c2 rows (16-bit).
+struct StreamWs {
+  int64_t nl, qhat, khat, total;
+};
+StreamWs stream_ws(const farope_attn_desc* d) {
+  const int64_t rows = (int64_t)d->batch * d->heads * d->seq_len;
+  auto al = [](int64_t x) { return (x + 63) & ~int64_t(63); };
+  StreamWs w{};
+  w.nl = al(rows);
+  w.qhat = al(w.nl + rows);
+  w.khat = al(w.qhat + rows * d->head_dim / 2);
+  w.total = w.khat + rows * d->head_dim / 2;
+  return w;
+}
+
 // Caller workspace of farope_attn_bwd: enough for whichever path the call
 // takes.
 int64_t bwd_caller_ws(const farope_attn_desc* d) {
   const int64_t s = split_caller_ws(d);
+  if (bwd_stream(d)) return stream_ws(d).total > s ? stream_ws(d).total : s;
   if (!ds_possible(d)) return s;
   const int64_t t = ds_ws(d).total;
   return t > s ? t : s;
@@ -404,6 +442,16 @@ int bwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
       p.vec_dk && p.vec_dv && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
       (!static_ws || ds_ws(desc).total <= kScratchFloats))
     return ds_pass(p, desc, delta_ws, st);
+  // streamed tiles (the static workspace only when all of it fits)
+  if (bwd_stream(desc) && p.vec_q && p.vec_k && p.vec_v && p.vec_o && p.vec_do && p.vec_dq &&
+      p.vec_dk && p.vec_dv && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
+      (!static_ws || stream_ws(desc).total <= kScratchFloats)) {
+    const StreamWs w = stream_ws(desc);
+    p.row_stat = delta_ws + w.nl;
+    p.qhat_f = delta_ws + w.qhat;
+    p.khat = delta_ws + w.khat;
+    return launch_rc(launch_bwd_stream(p, desc->io_dtype, D, st));
+  }
   // dQ (and delta, which the dK/dV pass reads for every row) before dK / dV
   if (key_from_dq(desc, p.vec_k && p.vec_v))
     p.xk_ws = delta_ws + (int64_t)desc->batch * desc->heads * desc->seq_len;
@@ -426,6 +474,57 @@ int bwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
     p.row_stat = delta_ws + stat_offset(desc);
   FAROPE_TRY(dq_pass(p, desc, true, st));
   return dkdv_pass(p, desc, st);
+}
+
+int fwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride[4],
+                    const void* k, const int64_t k_stride[4], const void* v,
+                    const int64_t v_stride[4], const float* rope_packed, size_t rope_elems, void* o,
+                    const int64_t o_stride[4], void* o_res, float* lse, float* ws, void* stream) {
+  FAROPE_TRY(check_desc(desc));
+  if (!q_stride || !k_stride || !v_stride || !o_stride) return FAROPE_ERR_NULL;
+  const int es = elem_size(desc->io_dtype);
+  FAROPE_TRY(check_ptr(q, es));
+  FAROPE_TRY(check_ptr(k, es));
+  FAROPE_TRY(check_ptr(v, es));
+  FAROPE_TRY(check_ptr(o, es));
+  FAROPE_TRY(check_ptr(lse, 4));
+  FAROPE_TRY(check_table(desc, rope_packed, rope_elems));
+  if (o_res) FAROPE_TRY(check_ptr(o_res, 16));
+  if (ws) FAROPE_TRY(check_ptr(ws, 16));
+
+  FwdParams p;
+  p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
+  p.o_res = o_residual(desc->io_dtype, desc->compute_dtype, desc->head_dim) ? o_res : nullptr;
+  copy4(p.sq, q_stride); copy4(p.sk, k_stride); copy4(p.sv, v_stride); copy4(p.so, o_stride);
+  p.rope = rope_packed;
+  p.B = desc->batch; p.H = desc->heads; p.N = desc->seq_len; p.has_cls = desc->has_cls;
+  p.scale_log2 = desc->softmax_scale * 1.4426950408889634f;
+  p.vec_q = vec_ok(q, q_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_k = vec_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_v = vec_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_o = vec_out_ok(o, o_stride, es, desc->seq_len, desc->head_dim);
+  const bool vec = p.vec_q && p.vec_k && p.vec_v && p.vec_o;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (fwd_plane(desc, vec)) {
+    p.n_blk = 1;
+    p.n_items = p.B * p.H;
+    p.x_rows = 0;
+    return launch_rc(launch_fwd_plane(p, desc->io_dtype, st));
+  }
+  if (ws && fwd_stream(desc) && vec) {
+    const KhatParams kp{k, ws, {k_stride[0], k_stride[1], k_stride[2]}, rope_packed, p.B * p.H, p.H, p.N, p.has_cls, p.scale_log2};
+    FAROPE_TRY(launch_rc(launch_stream_khat(kp, desc->compute_dtype, desc->head_dim, st)));
+    return launch_rc(launch_fwd_stream(p, ws, desc->io_dtype, desc->head_dim, st));
+  }
+  const int rows = fwd_block_rows(desc->head_dim, desc->io_dtype, desc->compute_dtype);
+  const int tail = tail_of(p.B * p.H, p.N, rows);
+  p.n_blk = main_blocks(p.B * p.H, p.N, rows);
+  p.n_items = p.B * p.H * p.n_blk;
+  p.x_rows = tail == 1 && fwd_folds_tail(desc->io_dtype, desc->compute_dtype, desc->head_dim, vec);
+  FAROPE_TRY(launch_rc(launch_fwd(p, desc->io_dtype, desc->compute_dtype, desc->head_dim, st)));
+  if (tail && !p.x_rows)
+    FAROPE_TRY(launch_rc(launch_fwd_tail(p, desc->io_dtype, desc->head_dim, p.N - tail, st)));
+  return FAROPE_OK;
 }
 
 }  // namespace
@@ -487,6 +586,11 @@ int farope_tile_config(const farope_attn_desc* desc, int32_t which, int32_t out[
     out[1] = rows;
     out[2] = main_blocks(desc->batch * desc->heads, N, rows);
     out[3] = fwd_threads(D);
+  } else if (bwd_stream(desc)) {
+    out[0] = BWD_STREAM;
+    out[1] = kStreamTileRows;
+    out[2] = cdiv(N, kStreamTileRows);
+    out[3] = kStreamThreads;
   } else {
     const bool fu = bwd_fused(desc);
     out[0] = fu ? BWD_FUSED : ds_possible(desc) ? BWD_DS : keys_possible(desc) ? BWD_SPLIT16 : BWD_SPLIT;
@@ -512,45 +616,19 @@ int farope_attn_fwd(const farope_attn_desc* desc, const void* q, const int64_t q
                     const void* k, const int64_t k_stride[4], const void* v,
                     const int64_t v_stride[4], const float* rope_packed, size_t rope_elems, void* o,
                     const int64_t o_stride[4], void* o_res, float* lse, void* stream) {
-  FAROPE_TRY(check_desc(desc));
-  if (!q_stride || !k_stride || !v_stride || !o_stride) return FAROPE_ERR_NULL;
-  const int es = elem_size(desc->io_dtype);
-  FAROPE_TRY(check_ptr(q, es));
-  FAROPE_TRY(check_ptr(k, es));
-  FAROPE_TRY(check_ptr(v, es));
-  FAROPE_TRY(check_ptr(o, es));
-  FAROPE_TRY(check_ptr(lse, 4));
-  FAROPE_TRY(check_table(desc, rope_packed, rope_elems));
-  if (o_res) FAROPE_TRY(check_ptr(o_res, 16));
+  return fwd_impl(desc, q, q_stride, k, k_stride, v, v_stride, rope_packed, rope_elems, o, o_stride, o_res, lse, nullptr, stream);
+}
 
-  FwdParams p;
-  p.q = q; p.k = k; p.v = v; p.o = o; p.lse = lse;
-  p.o_res = o_residual(desc->io_dtype, desc->compute_dtype, desc->head_dim) ? o_res : nullptr;
-  copy4(p.sq, q_stride); copy4(p.sk, k_stride); copy4(p.sv, v_stride); copy4(p.so, o_stride);
-  p.rope = rope_packed;
-  p.B = desc->batch; p.H = desc->heads; p.N = desc->seq_len; p.has_cls = desc->has_cls;
-  p.scale_log2 = desc->softmax_scale * 1.4426950408889634f;
-  p.vec_q = vec_ok(q, q_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_k = vec_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_v = vec_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_o = vec_out_ok(o, o_stride, es, desc->seq_len, desc->head_dim);
-  const bool vec = p.vec_q && p.vec_k && p.vec_v && p.vec_o;
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (fwd_plane(desc, vec)) {
-    p.n_blk = 1;
-    p.n_items = p.B * p.H;
-    p.x_rows = 0;
-    return launch_rc(launch_fwd_plane(p, desc->io_dtype, st));
-  }
-  const int rows = fwd_block_rows(desc->head_dim, desc->io_dtype, desc->compute_dtype);
-  const int tail = tail_of(p.B * p.H, p.N, rows);
-  p.n_blk = main_blocks(p.B * p.H, p.N, rows);
-  p.n_items = p.B * p.H * p.n_blk;
-  p.x_rows = tail == 1 && fwd_folds_tail(desc->io_dtype, desc->compute_dtype, desc->head_dim, vec);
-  FAROPE_TRY(launch_rc(launch_fwd(p, desc->io_dtype, desc->compute_dtype, desc->head_dim, st)));
-  if (tail && !p.x_rows)
-    FAROPE_TRY(launch_rc(launch_fwd_tail(p, desc->io_dtype, desc->head_dim, p.N - tail, st)));
-  return FAROPE_OK;
+size_t farope_attn_fwd_workspace_elems(const farope_attn_desc* desc) {
+  if (check_desc(desc) != FAROPE_OK || !fwd_stream(desc)) return 0;
+  return (size_t)desc->batch * desc->heads * desc->seq_len * desc->head_dim / 2;
+}
+
+int farope_attn_fwd_ws(const farope_attn_desc* desc, const void* q, const int64_t q_stride[4],
+                       const void* k, const int64_t k_stride[4], const void* v,
+                       const int64_t v_stride[4], const float* rope_packed, size_t rope_elems, void* o,
+                       const int64_t o_stride[4], void* o_res, float* lse, float* ws, void* stream) {
+  return fwd_impl(desc, q, q_stride, k, k_stride, v, v_stride, rope_packed, rope_elems, o, o_stride, o_res, lse, ws, stream);
 }
 
 int farope_attn_bwd_preprocess(const farope_attn_desc* desc, const void* o,

@@ -73,6 +73,8 @@ enum BwdVariant : int {
                     // (bwd_keys.hip; with vector access to every tensor, else BWD_SPLIT)
   BWD_DS = 3,       // row pass + key tiles that store dS + dQ as one GEMM over it
                     // (bwd_ds.hip; with vector access to every tensor, else BWD_SPLIT16)
+  BWD_STREAM = 4,   // streamed dQ tiles, then streamed dK/dV tiles (bwd_stream.hip;
+                    // with vector access to every tensor, else BWD_SPLIT)
 };
 
 // Launchers: return hipSuccess or the launch error.  io/ct are DT_* codes.
@@ -125,6 +127,25 @@ constexpr int kDsQueryRows = 256;   // query rows per dQ GEMM workgroup
 constexpr int kDsMaxKeyTiles = 256;  // key tiles per plane (N < 32768, from the 32-bit dS^T offsets)
 hipError_t launch_bwd_ds_prep(const BwdParams& p, int io, hipStream_t st);
 hipError_t launch_bwd_ds_dq(const BwdParams& p, int io, hipStream_t st);
+
+// Streamed-tile backward (bwd_stream.hip): p.delta, p.row_stat (-LSE2 rows),
+// p.qhat_f and p.khat are its workspace.
+constexpr int kStreamTileRows = 128;   // rows per workgroup (forward, dQ, dK/dV)
+constexpr int kStreamThreads = 256;
+// K-hat * c2 rows [planes][N][D] of 16-bit K (any vector-access strides), in
+// the compute type: what both passes stream.
+struct KhatParams {
+  const void* k;
+  void* khat;
+  int64_t sk[3];
+  const float* rope;
+  int planes, H, N, has_cls;
+  float c2;            // softmax_scale * log2(e)
+};
+hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st);
+// Forward over 128-query tiles; khat from launch_stream_khat.
+hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st);
+hipError_t launch_bwd_stream(const BwdParams& p, int io, int D, hipStream_t st);
 
 // Whether the forward block kernel computes a single tail row itself
 // (FwdParams::x_rows = 1) instead of launch_fwd_tail: fp16 logit operands with
