@@ -14,6 +14,7 @@ import threading
 import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libfarope.so")
+OPS_PATH = os.path.join(os.path.dirname(LIB_PATH), "libfarope_torch.so")   # the torch ops' GPU kernels
 
 F32, F16, BF16 = 0, 1, 2
 DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
@@ -116,6 +117,38 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = args
             _lib = lib
     return _lib
+
+
+_ops_error: str | None = None
+
+
+def load_torch_ops() -> None:
+    """Register the GPU kernels of farope::attn_fwd / attn_bwd (csrc/torch_ops.cpp).
+
+    A missing or unloadable library is remembered, not raised: importing (and
+    building) the package needs no library, GPU calls do (require_torch_ops).
+    """
+    global _ops_error
+    try:
+        torch.ops.load_library(OPS_PATH)
+        _ops_error = None
+    except OSError as e:
+        _ops_error = str(e)
+
+
+def ops_error() -> str | None:
+    """Why the ops library could not be loaded (None: it is)."""
+    return _ops_error
+
+
+def require_torch_ops() -> None:
+    """Raise: a GPU call reached the ops' Python body, so their GPU kernels are missing."""
+    load()
+    why = f": {_ops_error}" if _ops_error else ""
+    raise RuntimeError(
+        f"farope: the GPU kernels of the torch ops are not loaded from {OPS_PATH}{why}; build them with "
+        "`python -m triton_fused_rope_flash_attn_amd.build` (or __graft_entry__.build())"
+    )
 
 
 def strerror(rc: int) -> str:

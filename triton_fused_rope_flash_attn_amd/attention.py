@@ -14,8 +14,9 @@ and reused by backward (FA:1061).
 
 The work is done by two ``torch.library`` custom ops, ``farope::attn_fwd``
 -> (O, LSE) and ``farope::attn_bwd`` -> (dQ, dK, dV), each a single call into
-libfarope.so on the current HIP stream.  Both have fake (meta) kernels, so
-the ops are opaque but traceable under ``torch.compile``.  There is no CPU
+libfarope.so on the current HIP stream, made by native kernels of the ops
+(libfarope_torch.so).  Both have fake (meta) kernels, so the ops are opaque but
+traceable under ``torch.compile``.  There is no CPU
 or eager-PyTorch fallback: CPU tensors raise.
 """
 from __future__ import annotations
@@ -98,18 +99,7 @@ def attn_fwd(
     _check_qkv(q, k, v)
     B, H, N, D = q.shape
     _check_rope(rope, n_pos, D, q.device)
-    o = torch.empty((B, H, N, D), dtype=q.dtype, device=q.device)
-    lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device)
-    io = _lib.DTYPE_CODE[q.dtype]
-    res = _uses_residual(io, compute_dtype, D)
-    o_res = torch.empty((B, H, N, D) if res else (0,), dtype=q.dtype, device=q.device)
-    desc = _lib.make_desc(B, H, N, D, n_pos, has_cls, io, compute_dtype, softmax_scale)
-    # rotated K rows of the streamed forward (none for the other kernels)
-    elems = _lib.fwd_workspace_elems(desc)
-    ws = torch.empty(elems, dtype=torch.float32, device=q.device) if elems else None
-    with torch.cuda.device(q.device):
-        _lib.attn_fwd(desc, q, k, v, rope, o, lse, o_res, ws)
-    return o, lse, o_res
+    _lib.require_torch_ops()   # (GPU tensors run the native kernel, see below)
 
 
 @attn_fwd.register_fake
@@ -142,27 +132,7 @@ def attn_bwd(
     _check_qkv(q, k, v)
     B, H, N, D = q.shape
     _check_rope(rope, n_pos, D, q.device)
-    if do.shape != q.shape or o.shape != q.shape:
-        raise ValueError("farope: dO and O must have Q's shape")
-    if do.dtype != q.dtype:
-        do = do.to(q.dtype)
-    if lse.dtype != torch.float32 or lse.shape != (B, H, N) or not lse.is_contiguous():
-        raise ValueError("farope: LSE must be contiguous fp32 [B, H, N]")
-    dq = torch.empty((B, H, N, D), dtype=q.dtype, device=q.device)
-    dk = torch.empty((B, H, N, D), dtype=k.dtype, device=q.device)
-    dv = torch.empty((B, H, N, D), dtype=v.dtype, device=q.device)
-    desc = _lib.make_desc(B, H, N, D, n_pos, has_cls, _lib.DTYPE_CODE[q.dtype], compute_dtype,
-                          softmax_scale)
-    # the backward's workspace (delta rows, and at head_dim 128 the rotated Q
-    # rows, row statistics and stored dS^T of the key tiles); none for the
-    # one-pass backward, which keeps delta on chip
-    ws = _lib.bwd_workspace_elems(desc)
-    delta = torch.empty(ws, dtype=torch.float32, device=q.device) if ws else None
-    if o_res.numel() and (o_res.shape != q.shape or o_res.dtype != q.dtype or not o_res.is_contiguous()):
-        raise ValueError("farope: O_res must be contiguous with Q's shape and dtype, or empty")
-    with torch.cuda.device(q.device):
-        _lib.attn_bwd(desc, q, k, v, o, do, lse, rope, dq, dk, dv, delta, o_res)
-    return dq, dk, dv
+    _lib.require_torch_ops()
 
 
 @attn_bwd.register_fake
@@ -195,6 +165,11 @@ def _fwd_backward(ctx, do, _dlse, _dres):
 
 
 attn_fwd.register_autograd(_fwd_backward, setup_context=_fwd_setup_context)
+
+# The ops' kernels and autograd for GPU tensors are native (csrc/torch_ops.cpp):
+# registered for the CUDA dispatch keys, they take precedence over the bodies
+# above, which are left with CPU tensors (they raise) and meta tensors.
+_lib.load_torch_ops()
 
 
 # ---------------------------------------------------------------------------

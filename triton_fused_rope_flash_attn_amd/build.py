@@ -1,8 +1,9 @@
-"""Build recipe for libfarope.so (hand-written gfx950 HIP kernels + C ABI).
+"""Build recipe for libfarope.so (hand-written gfx950 HIP kernels + C ABI) and
+libfarope_torch.so (the torch ops' GPU kernels over it, host code).
 
-Compiles every translation unit under csrc/ with hipcc for gfx950 (in
-parallel), then links one shared library next to this file, where
-``_lib.py`` loads it.  Runs on a machine without a GPU: hipcc
+Compiles every HIP translation unit under csrc/ with hipcc for gfx950 (in
+parallel), then links the shared libraries next to this file, where
+``_lib.py`` loads them.  Runs on a machine without a GPU: hipcc
 cross-compiles.  ``python -m triton_fused_rope_flash_attn_amd.build``.
 """
 from __future__ import annotations
@@ -26,6 +27,8 @@ SOURCES = ["api.hip", "fwd.hip", "fwd_plane.hip", "fwd_stream.hip", "bwd.hip", "
 # fragments in AGPRs.
 EXTRA_FLAGS = {"fwd_plane.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 ARCH = "gfx950"
+OPS_SOURCE = "torch_ops.cpp"
+OPS_PATH = os.path.join(PKG_DIR, "libfarope_torch.so")
 
 
 def _hipcc() -> str:
@@ -64,8 +67,25 @@ def _run(cmd: list[str]) -> None:
         raise RuntimeError(f"command failed ({res.returncode}): {' '.join(cmd)}\n{out}")
 
 
+def ops_commands(obj: str, out: str) -> list[list[str]]:
+    """Compile and link commands of the torch ops library (host code against
+    torch's headers; it finds libfarope.so next to itself)."""
+    import torch
+
+    tdir = os.path.dirname(torch.__file__)
+    hipcc = _hipcc()
+    rocm_inc = os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(hipcc))), "include")
+    compile_ = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                f"-I{INCLUDE}", f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include", f"-I{rocm_inc}",
+                "-Wno-deprecated-declarations", "-c", os.path.join(CSRC, OPS_SOURCE), "-o", obj]
+    link = [hipcc, "-shared", "-fPIC", obj, "-o", out, f"-L{PKG_DIR}", "-l:" + LIB_NAME, f"-L{tdir}/lib",
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-Wl,-rpath,$ORIGIN"]
+    return [compile_, link]
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> str:
-    """Compile and link libfarope.so; returns its path."""
+    """Compile and link libfarope.so and libfarope_torch.so; returns the former's path."""
     hipcc = _hipcc()
     flags = compile_flags()
     tmp = tempfile.mkdtemp(prefix="farope_build_")
@@ -76,6 +96,9 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
             obj = os.path.join(tmp, src.replace(".hip", ".o"))
             objs.append(obj)
             cmds.append([hipcc, *flags, *EXTRA_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj])
+        ops_obj, ops_out = os.path.join(tmp, "torch_ops.o"), OPS_PATH + ".tmp"
+        ops_compile, ops_link = ops_commands(ops_obj, ops_out)
+        cmds.append(ops_compile)
         jobs = jobs or min(len(cmds), os.cpu_count() or 1, 16)
         with _cf.ThreadPoolExecutor(max_workers=jobs) as ex:
             for cmd, fut in zip(cmds, [ex.submit(_run, c) for c in cmds]):
@@ -85,10 +108,12 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
         out_tmp = LIB_PATH + ".tmp"
         _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", out_tmp])
         os.replace(out_tmp, LIB_PATH)
+        _run(ops_link)
+        os.replace(ops_out, OPS_PATH)
     finally:
         shutil.rmtree(tmp, ignore_errors=True)
     if verbose:
-        print(f"built {LIB_PATH}", flush=True)
+        print(f"built {LIB_PATH} and {OPS_PATH}", flush=True)
     return LIB_PATH
 
 
