@@ -1,0 +1,65 @@
+"""GPU: the short-plane kernels (csrc/short.hip) against the fp32 oracle."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import torch_ref
+from tests.cases import ROPE_BASE, TOL_MEAN
+from tests.test_gpu_parity import _compare
+from triton_fused_rope_flash_attn_amd import CosSinTable, _lib
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DT = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32, "amp": torch.float32}
+
+
+def _nan(*shape, dtype=torch.float32):
+    return torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+
+
+# both sides of the 32-row blocks, the 64-row tiles, the staged 64 / 128 / 256
+# rows and the longest plane: N = 4 (less than a subtile), 10, 36, 49, 64, 65, 82,
+# 121, 122, 145, 197, 225, 226, 256; few planes, so that every rule takes them
+@pytest.mark.parametrize("side,has_cls", [(2, False), (3, True), (6, False), (7, False), (8, False), (8, True), (9, True),
+                                          (11, False), (11, True), (12, True), (14, True), (15, False), (15, True),
+                                          (16, False)])
+@pytest.mark.parametrize("D,io", [(64, "bf16"), (32, "fp16"), (32, "amp"), (64, "fp32"), (64, "amp"), (32, "fp32")])
+def test_short_planes(side, has_cls, D, io):
+    B, H = 2, 3
+    N = side * side + int(has_cls)
+    dt = DT[io]
+    print(f"short planes N={N} D={D} {io}", flush=True)
+    g = torch.Generator().manual_seed(61)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    # views of one projection buffer; dO a transposed view
+    q, k, v = torch.randn(B, N, 3, H, D, generator=g).to(dt).to(DEV).permute(2, 0, 3, 1, 4).unbind(0)
+    do = torch.randn(B, N, H, D, generator=g).to(dt).to(DEV).transpose(1, 2)
+    comp = _lib.BF16 if io == "amp" else _lib.DTYPE_CODE[dt]
+    desc = _lib.make_desc(B, H, N, D, N - int(has_cls), has_cls, _lib.DTYPE_CODE[dt], comp, D ** -0.5)
+    rope = table.packed()
+
+    def run():
+        o, dq, dk, dv = (_nan(B, H, N, D, dtype=dt) for _ in range(4))
+        lse = _nan(B, H, N)
+        _lib.attn_fwd(desc, q, k, v, rope, o, lse)
+        _lib.attn_bwd(desc, q, k, v, o, do, lse, rope, dq, dk, dv, _nan(max(_lib.bwd_workspace_elems(desc), 1)))
+        torch.cuda.synchronize()
+        return o, lse, dq, dk, dv
+
+    got = run()
+    ref = torch_ref.forward_backward(*(t.float() for t in (q, k, v, do)), *table.tables(), has_cls)
+    lse = torch_ref.logsumexp_rows(q.float(), k.float(), *table.tables(), has_cls)
+    if io == "fp32":
+        _compare(f"short-fp32-N{N}-D{D}", (got[0], *got[2:]), ref, tol_max=1e-4, tol_mean=1e-5)
+    else:
+        # fp32 tensors computed in bf16 are held to bf16's bound, the mean to twice it: the
+        # oracle's inputs are not bf16 there, so up to four operands of a product
+        # (dO, V, K-hat, dS) are off by 2^-9 each, and the gradients of a plane of a few
+        # keys have a mean size of 0.3 (4 * 2^-9 * 0.3 = 2.3e-3)
+        amp = io == "amp"
+        _compare(f"short-{io}-N{N}-D{D}", (got[0], *got[2:]), ref, tol_mean=2e-3 if amp else TOL_MEAN,
+                 out_dtype=torch.bfloat16 if amp else dt)
+    # a logit of size s is off by about 2^-8 s (bf16 operands)
+    assert (got[1] - lse).abs().max().item() < (1e-4 if io == "fp32" else 2e-2)
+    assert all(torch.equal(a, b) for a, b in zip(got, run()))

@@ -335,6 +335,55 @@ bool fwd_stream(const farope_attn_desc* d) { return stream_shape(d) && d->seq_le
 bool bwd_stream(const farope_attn_desc* d) {
   return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim == 64 ? 1 : 0);
 }
+// The short-plane kernels (short.hip): tensors in the compute type or in fp32,
+// head_dim 32 or 64, N <= 256.  (Vector access to every tensor is checked at
+// the call.)  short_tiles: their 64-row tiles over the whole call.
+bool short_shape(const farope_attn_desc* d) {
+  if (d->io_dtype != FAROPE_F32 && d->io_dtype != d->compute_dtype) return false;
+  if (d->head_dim != 64 && d->head_dim != 32) return false;
+  return d->seq_len <= kPlaneMaxN && (int64_t)d->batch * d->heads * 2 * cdiv(d->seq_len, kShortTileRows) <= INT32_MAX;
+}
+int64_t short_tiles(const farope_attn_desc* d) {
+  return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kShortTileRows);
+}
+// Forward: up to 128 rows always, longer planes while the call has too few of
+// them to fill the chip with one workgroup (fwd_kernel) or one wave
+// (fwd_plane) a plane, whose time hardly changes up to 256 or 1024 planes.
+// Measured (us, those kernels / short; "planes x N"): bf16 D 64: 3072 x 122
+// 58 / 42, 144 x 121 8.9 / 7.6; fwd_plane 12 x 197 22.6 / 7.2, 96 23.0 / 8.3,
+// 384 26.0 / 21.9, 576 27.4 / 31.9; fwd_kernel 120 x 144 10.5 / 7.9, 192 x 144
+// 10.7 / 11.5, 120 x 256 12.4 / 8.5, 384 x 256 22.3 / 23.0; fp32 compute 96 x
+// 197 26.6 / 18.8, 192 28.1 / 28.7.  D 32: 4096 x 64 42 / 14, 4096 x 144 76 / 61,
+// 512 x 197 14.3 / 14.0, 4096 x 197 84 / 87; fp32 compute 512 x 197 29.9 / 30.1,
+// 4096 x 144 162 / 168.
+bool fwd_short(const farope_attn_desc* d) {
+  if (!short_shape(d)) return false;
+  if (d->seq_len <= 128) return true;
+  const int64_t t = short_tiles(d);
+  const bool f32 = d->compute_dtype == FAROPE_F32;
+  if (d->head_dim == 32) return f32 ? t <= 1024 : d->seq_len <= 192 || t <= 2048;
+  return t <= (fwd_plane(d, true) ? 1536 : 512);
+}
+// Backward.  fp32 compute, and 16-bit tensors at head_dim 32: always (it
+// replaces two kernels of 128-row tiles).  16-bit compute at head_dim 64: 33 to
+// 64 rows in 16-bit tensors always; else against the one-pass kernel while two
+// workgroups a CU hold the whole call (with N <= 32 that kernel's delta is the
+// more exact one and stays); fp32 tensors likewise, at head_dim 32 up to 64
+// rows always.  Measured (us, those kernels / short): fp32 compute, D 64: 16 x
+// 197 54.7 / 15.6, 1536 x 197 731 / 607, 1536 x 64 151 / 53; D 32 4096 x 144 682
+// / 350.  bf16 D 32: 4096 x 64 75 / 34, 4096 x 197 270 / 257, 4096 x 256 303 /
+// 302.  bf16 D 64: 3072 x 64 60.6 / 56.0, 12 x 197 16.9 / 9.2, 48 x 197 17.3 /
+// 11.7, 96 x 197 17.6 / 17.6, 192 x 197 18.1 / 29.0.  fp32 tensors in bf16: D 32
+// 4096 x 64 97 / 67, 1024 x 197 82 / 97; D 64 48 x 197 26.0 / 17.9, 3072 x 64
+// 91 / 113.
+bool bwd_short(const farope_attn_desc* d) {
+  if (!short_shape(d)) return false;
+  if (d->compute_dtype == FAROPE_F32) return true;
+  const bool io16 = d->io_dtype != FAROPE_F32, one = d->seq_len <= kShortTileRows;
+  if (d->head_dim == 64 && d->seq_len <= 32) return false;
+  if (d->head_dim == 32 ? io16 || one : io16 && one) return true;
+  return 2 * short_tiles(d) <= 512;
+}
 // Its workspace, in fp32 elements, each part from a 256-byte boundary:
 // -delta rows, -LSE2 rows, Q-hat rows and K-hat * c2 rows (16-bit).
 struct StreamWs {
@@ -433,6 +482,8 @@ int bwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
   p.vec_dv = vec_out_ok(dv, dv_stride, es, desc->seq_len, desc->head_dim);
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int D = desc->head_dim;
+  if (bwd_short(desc) && p.vec_q && p.vec_k && p.vec_v && p.vec_o && p.vec_do && p.vec_dq && p.vec_dk && p.vec_dv)
+    return launch_rc(launch_bwd_short(p, desc->io_dtype, desc->compute_dtype, D, st));
   if (fused) {
     p.n_blk = 1;
     return launch_rc(launch_bwd_fused(p, desc->io_dtype, desc->compute_dtype, st));
@@ -505,6 +556,8 @@ int fwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
   p.vec_o = vec_out_ok(o, o_stride, es, desc->seq_len, desc->head_dim);
   const bool vec = p.vec_q && p.vec_k && p.vec_v && p.vec_o;
   const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (fwd_short(desc) && vec)
+    return launch_rc(launch_fwd_short(p, desc->io_dtype, desc->compute_dtype, desc->head_dim, st));
   if (fwd_plane(desc, vec)) {
     p.n_blk = 1;
     p.n_items = p.B * p.H;

@@ -147,6 +147,12 @@ hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st
 hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st);
 hipError_t launch_bwd_stream(const BwdParams& p, int io, int D, hipStream_t st);
 
+// Short planes (short.hip): head_dim 32 or 64, N <= 256, 16-bit compute, vector
+// access to every tensor; 64 rows per workgroup, the backward in one launch.
+constexpr int kShortTileRows = 64;
+hipError_t launch_fwd_short(const FwdParams& p, int io, int ct, int D, hipStream_t st);
+hipError_t launch_bwd_short(const BwdParams& p, int io, int ct, int D, hipStream_t st);
+
 // Whether the forward block kernel computes a single tail row itself
 // (FwdParams::x_rows = 1) instead of launch_fwd_tail: fp16 logit operands with
 // vector access (vec: every tensor of the call allows it).
