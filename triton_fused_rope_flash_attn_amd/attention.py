@@ -43,6 +43,13 @@ def _sdpa_comp_dtype(x: torch.Tensor) -> torch.dtype:
     raise TypeError(f"farope: unsupported compute dtype {dtype} (float16, bfloat16, float32)")
 
 
+def _check_device(t: torch.Tensor) -> None:
+    if not t.is_cuda:
+        raise RuntimeError(
+            f"farope runs on ROCm GPUs only (hand-written gfx950 kernels); got a {t.device} tensor"
+        )
+
+
 def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
     if q.dim() != 4:
         raise ValueError(f"Q must be [B, H, N, D]; got shape {tuple(q.shape)}")
@@ -54,10 +61,7 @@ def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
         raise TypeError(f"farope: unsupported tensor dtype {q.dtype}")
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise TypeError(f"farope: Q, K, V must share one dtype; got {q.dtype}, {k.dtype}, {v.dtype}")
-    if not q.is_cuda:
-        raise RuntimeError(
-            f"farope runs on ROCm GPUs only (hand-written gfx950 kernels); got a {q.device} tensor"
-        )
+    _check_device(q)
     if k.device != q.device or v.device != q.device:
         raise RuntimeError("farope: Q, K, V must be on the same device")
 
@@ -166,6 +170,62 @@ def _fwd_backward(ctx, do, _dlse, _dres):
 
 attn_fwd.register_autograd(_fwd_backward, setup_context=_fwd_setup_context)
 
+
+# Packed layout (an attention layer's): q, k, v as thirds of one projection
+# output qkv [B, N, 3 H D], O as [B, N, H D]; dqkv comes back as one tensor.
+@torch.library.custom_op("farope::attn_qkv_fwd", mutates_args=())
+def attn_qkv_fwd(qkv: torch.Tensor, rope: torch.Tensor, heads: int, n_pos: int, has_cls: bool,
+                 softmax_scale: float, compute_dtype: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """-> (O [B, N, H D], LSE, O_res), as attn_fwd."""
+    _check_device(qkv)
+    _lib.require_torch_ops()
+
+
+@attn_qkv_fwd.register_fake
+def _attn_qkv_fwd_fake(qkv, rope, heads, n_pos, has_cls, softmax_scale, compute_dtype):
+    B, N, C3 = qkv.shape
+    D = C3 // (3 * heads)
+    res = _uses_residual(_lib.DTYPE_CODE.get(qkv.dtype, -1), compute_dtype, D)
+    return (
+        qkv.new_empty((B, N, heads * D)),
+        qkv.new_empty((B, heads, N), dtype=torch.float32),
+        qkv.new_empty((B, heads, N, D) if res else (0,)),
+    )
+
+
+@torch.library.custom_op("farope::attn_qkv_bwd", mutates_args=())
+def attn_qkv_bwd(do: torch.Tensor, qkv: torch.Tensor, o: torch.Tensor, lse: torch.Tensor, rope: torch.Tensor,
+                 heads: int, n_pos: int, has_cls: bool, softmax_scale: float, compute_dtype: int,
+                 o_res: torch.Tensor) -> torch.Tensor:
+    """-> dqkv [B, N, 3 H D]."""
+    _check_device(qkv)
+    _lib.require_torch_ops()
+
+
+@attn_qkv_bwd.register_fake
+def _attn_qkv_bwd_fake(do, qkv, o, lse, rope, heads, n_pos, has_cls, softmax_scale, compute_dtype, o_res):
+    return qkv.new_empty(tuple(qkv.shape))
+
+
+def _qkv_setup_context(ctx, inputs, output):
+    qkv, rope, ctx.heads, ctx.n_pos, ctx.has_cls, ctx.softmax_scale, ctx.compute_dtype = inputs
+    o, lse, o_res = output
+    ctx.mark_non_differentiable(lse, o_res)
+    ctx.set_materialize_grads(False)
+    ctx.save_for_backward(qkv, o, lse, rope, o_res)
+
+
+def _qkv_backward(ctx, do, _dlse, _dres):
+    if do is None:
+        return (None,) * 7
+    qkv, o, lse, rope, o_res = ctx.saved_tensors
+    dqkv = attn_qkv_bwd(do, qkv, o, lse, rope, ctx.heads, ctx.n_pos, ctx.has_cls, ctx.softmax_scale,
+                        ctx.compute_dtype, o_res)
+    return dqkv, None, None, None, None, None, None
+
+
+attn_qkv_fwd.register_autograd(_qkv_backward, setup_context=_qkv_setup_context)
+
 # The ops' kernels and autograd for GPU tensors are native (csrc/torch_ops.cpp):
 # registered for the CUDA dispatch keys, they take precedence over the bodies
 # above, which are left with CPU tensors (they raise) and meta tensors.
@@ -194,9 +254,8 @@ def rope_operand(cos_sin, n_pos: int, head_dim: int, device) -> torch.Tensor:
     return pack_rope_tables(cosp, sinp)
 
 
-def _prepare(Q, K, V, cos_sin, H_img, has_cls):
-    """Checks of TritonAttention.forward (FA:1014-1024) plus device/dtype checks."""
-    BATCH_SIZE, NUM_HEADS, SEQ_LEN, HEAD_DIM = Q.size()
+def _check_seq(SEQ_LEN, HEAD_DIM, H_img, has_cls):
+    """Checks of TritonAttention.forward (FA:1014-1024)."""
     assert (HEAD_DIM % 4) == 0, "HEAD_DIM must be divisible by 4 (2D RoPE requires pairs)."
     N_img = H_img ** 2
     if has_cls:
@@ -207,11 +266,38 @@ def _prepare(Q, K, V, cos_sin, H_img, has_cls):
         assert SEQ_LEN == N_img, (
             f"SEQ_LEN must equal H_img*W_img when has_cls=False (got {SEQ_LEN} vs {N_img})."
         )
+    return N_img
+
+
+def _prepare(Q, K, V, cos_sin, H_img, has_cls):
+    """The reference's checks plus device/dtype checks."""
+    BATCH_SIZE, NUM_HEADS, SEQ_LEN, HEAD_DIM = Q.size()
+    N_img = _check_seq(SEQ_LEN, HEAD_DIM, H_img, has_cls)
     _check_qkv(Q, K, V)
     comp = _sdpa_comp_dtype(Q)
     softmax_scale = 1.0 / (HEAD_DIM ** 0.5)
     rope = rope_operand(cos_sin, N_img, HEAD_DIM, Q.device)
     return rope, N_img, bool(has_cls), softmax_scale, _lib.DTYPE_CODE[comp]
+
+
+def packed_attention(qkv: torch.Tensor, cos_sin, num_heads: int, H_img: int, has_cls: bool) -> torch.Tensor:
+    """``sdpa_triton_fa_rope`` on the q, k, v of one projection output.
+
+    qkv: ``[B, N, 3 * num_heads * head_dim]`` with channels ordered (q | k | v,
+    head, channel); returns ``[B, N, num_heads * head_dim]``.  The same values
+    as on the strided views of ``qkv``, without the copies around them: O is
+    written where the output projection reads it, and the gradients where the
+    qkv projection's backward reads them.
+    """
+    B, N, C3 = qkv.shape
+    D = C3 // (3 * num_heads)
+    n_pos = _check_seq(N, D, H_img, has_cls)
+    if qkv.dtype not in _lib.DTYPE_CODE:
+        raise TypeError(f"farope: unsupported tensor dtype {qkv.dtype}")
+    _check_device(qkv)
+    comp = _sdpa_comp_dtype(qkv)
+    rope = rope_operand(cos_sin, n_pos, D, qkv.device)
+    return attn_qkv_fwd(qkv, rope, num_heads, n_pos, bool(has_cls), 1.0 / (D ** 0.5), _lib.DTYPE_CODE[comp])[0]
 
 
 class TritonAttention(torch.autograd.Function):

@@ -2,9 +2,9 @@
 
 ``RoPEAttention`` is the attention half of a ViT block as the reference's
 README benchmarks it (README:142-159, a ``vit_small_patch16_rope_224``-style
-model): ``qkv`` Linear -> ``[B, N, 3, H, D]`` -> q, k, v as strided views of
-that one buffer (no copies; the kernels take any strides, FA:1043) -> fused
-2D-RoPE attention -> ``[B, N, C]`` -> ``proj`` Linear.  The RoPE tables are
+model): ``qkv`` Linear -> ``[B, N, 3, H, D]`` -> fused 2D-RoPE attention on the
+q, k, v in that one buffer (no copies; the kernels take any strides, FA:1043)
+-> ``[B, N, C]`` -> ``proj`` Linear.  The RoPE tables are
 a ``CosSinTable`` submodule, so ``state_dict`` carries ``rope.COSP`` /
 ``rope.SINP`` as the reference's buffers.
 """
@@ -14,7 +14,7 @@ from typing import Callable, Optional
 
 import torch
 
-from .attention import sdpa_triton_fa_rope
+from .attention import packed_attention, sdpa_triton_fa_rope
 from .rope import CosSinTable
 
 __all__ = ["RoPEAttention"]
@@ -51,7 +51,12 @@ class RoPEAttention(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         B, N, C = x.shape
-        qkv = self.qkv(x).view(B, N, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
+        qkv = self.qkv(x)
+        if self.attn is sdpa_triton_fa_rope:
+            # the kernels read and write the projections' own layouts: the views
+            # below cost a copy of O and two of the gradients (64 x 197 x 384: 66 us)
+            return self.proj(packed_attention(qkv, self.rope, self.num_heads, self.H_img, self.has_cls))
+        qkv = qkv.view(B, N, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
         q, k, v = qkv.unbind(0)   # [B, H, N, D] views with strides (N*3C, D, 3C, 1)
         o = self.attn(q, k, v, self.rope, H_img=self.H_img, has_cls=self.has_cls)
         return self.proj(o.transpose(1, 2).reshape(B, N, C))

@@ -1,4 +1,5 @@
-// Native kernels of the torch ops farope::attn_fwd and farope::attn_bwd.
+// Native kernels of the torch ops farope::attn_fwd, farope::attn_bwd and their
+// packed-layout forms farope::attn_qkv_fwd, farope::attn_qkv_bwd.
 //
 // The ops, their schemas, fake kernels and CPU errors are defined in
 // attention.py.  This library adds their GPU kernels (dispatch keys CUDA and
@@ -65,18 +66,19 @@ void check_rope(const Tensor& rope, int64_t n_pos, int64_t d, const at::Device& 
   TORCH_CHECK(rope.device() == device, "farope: RoPE table on ", rope.device(), ", tensors on ", device);
 }
 
-farope_attn_desc make_desc(const Tensor& q, int64_t n_pos, bool has_cls, double scale, int64_t comp) {
+farope_attn_desc make_desc(int64_t B, int64_t H, int64_t N, int64_t D, at::ScalarType io, int64_t n_pos, bool has_cls,
+                           double scale, int64_t comp) {
   // (sizes past 32 bits are refused, not wrapped)
-  for (int64_t s : {q.size(0), q.size(1), q.size(2), q.size(3), n_pos, comp})
+  for (int64_t s : {B, H, N, D, n_pos, comp})
     TORCH_CHECK_VALUE(s >= 0 && s <= INT32_MAX, "farope: sizes must fit 32 bits");
   farope_attn_desc d;
-  d.batch = (int32_t)q.size(0);
-  d.heads = (int32_t)q.size(1);
-  d.seq_len = (int32_t)q.size(2);
-  d.head_dim = (int32_t)q.size(3);
+  d.batch = (int32_t)B;
+  d.heads = (int32_t)H;
+  d.seq_len = (int32_t)N;
+  d.head_dim = (int32_t)D;
   d.n_pos = (int32_t)n_pos;
   d.has_cls = has_cls ? 1 : 0;
-  d.io_dtype = dtype_code(q.scalar_type());
+  d.io_dtype = dtype_code(io);
   d.compute_dtype = (int32_t)comp;
   d.softmax_scale = (float)scale;
   return d;
@@ -100,7 +102,7 @@ Three attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& 
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
   check_rope(rope, n_pos, D, q.device());
   const c10::DeviceGuard guard(q.device());
-  const farope_attn_desc desc = make_desc(q, n_pos, has_cls, scale, comp);
+  const farope_attn_desc desc = make_desc(B, H, N, D, q.scalar_type(), n_pos, has_cls, scale, comp);
   const Tensor o = at::empty({B, H, N, D}, q.options());
   const Tensor lse = at::empty({B, H, N}, q.options().dtype(at::kFloat));
   const bool res = farope_attn_residual_elems(&desc) != 0;
@@ -131,7 +133,7 @@ Three attn_bwd(const Tensor& dout, const Tensor& q, const Tensor& k, const Tenso
                                        o_res.is_contiguous()),
                     "farope: O_res must be contiguous with Q's shape and dtype, or empty");
   const c10::DeviceGuard guard(q.device());
-  const farope_attn_desc desc = make_desc(q, n_pos, has_cls, scale, comp);
+  const farope_attn_desc desc = make_desc(B, H, N, D, q.scalar_type(), n_pos, has_cls, scale, comp);
   const Tensor dq = at::empty({B, H, N, D}, q.options());
   const Tensor dk = at::empty({B, H, N, D}, q.options());
   const Tensor dv = at::empty({B, H, N, D}, q.options());
@@ -142,6 +144,76 @@ Three attn_bwd(const Tensor& dout, const Tensor& q, const Tensor& k, const Tenso
                            dv.data_ptr(), strides(dv), floats(ws), stream_of(q)),
            "farope_attn_bwd");
   return {dq, dk, dv};
+}
+
+// ---------------------------------------------------------------------------
+// Packed layout: q, k, v are thirds of one [B, N, 3 H D] projection output and
+// O is [B, N, H D], as an attention layer's two projections hold them.  The
+// kernels read and write those places directly, so neither pass copies.
+// ---------------------------------------------------------------------------
+struct Heads {   // [B, H, N, D] view of part `third` of a [B, N, parts H D] tensor
+  void* ptr;
+  int64_t st[4];
+  Heads(const Tensor& t, int64_t third, int64_t H, int64_t D)
+      : ptr(static_cast<char*>(t.data_ptr()) + third * H * D * t.stride(2) * (int64_t)t.element_size()),
+        st{t.stride(0), D * t.stride(2), t.stride(1), t.stride(2)} {}
+};
+
+int64_t check_packed(const Tensor& qkv, const Tensor& rope, int64_t heads, int64_t n_pos) {
+  TORCH_CHECK_VALUE(qkv.dim() == 3 && heads > 0 && qkv.size(2) % (3 * heads) == 0,
+                    "farope: qkv must be [B, N, 3 * heads * head_dim]; got ", shape_str(qkv), " for ", heads, " heads");
+  TORCH_CHECK_TYPE(dtype_code(qkv.scalar_type()) >= 0, "farope: unsupported tensor dtype ", dtype_str(qkv));
+  TORCH_CHECK(qkv.is_cuda(), "farope runs on ROCm GPUs only (hand-written gfx950 kernels); got a ", qkv.device(), " tensor");
+  const int64_t D = qkv.size(2) / (3 * heads);
+  check_rope(rope, n_pos, D, qkv.device());
+  return D;
+}
+
+Three attn_qkv_fwd(const Tensor& qkv, const Tensor& rope, int64_t heads, int64_t n_pos, bool has_cls, double scale,
+                   int64_t comp) {
+  const int64_t D = check_packed(qkv, rope, heads, n_pos), B = qkv.size(0), N = qkv.size(1);
+  const c10::DeviceGuard guard(qkv.device());
+  const farope_attn_desc desc = make_desc(B, heads, N, D, qkv.scalar_type(), n_pos, has_cls, scale, comp);
+  const Tensor out = at::empty({B, N, heads * D}, qkv.options());
+  const Tensor lse = at::empty({B, heads, N}, qkv.options().dtype(at::kFloat));
+  const bool res = farope_attn_residual_elems(&desc) != 0;
+  const Tensor o_res = res ? at::empty({B, heads, N, D}, qkv.options()) : at::empty({0}, qkv.options());
+  const Tensor ws = workspace(qkv, farope_attn_fwd_workspace_elems(&desc));
+  const Heads q(qkv, 0, heads, D), k(qkv, 1, heads, D), v(qkv, 2, heads, D), o(out, 0, heads, D);
+  check_rc(farope_attn_fwd_ws(&desc, q.ptr, q.st, k.ptr, k.st, v.ptr, v.st, floats(rope), (size_t)rope.numel(), o.ptr, o.st,
+                              data(o_res), lse.data_ptr<float>(), floats(ws), stream_of(qkv)),
+           "farope_attn_fwd");
+  return {out, lse, o_res};
+}
+
+Tensor attn_qkv_bwd(const Tensor& dout, const Tensor& qkv, const Tensor& out, const Tensor& lse, const Tensor& rope,
+                    int64_t heads, int64_t n_pos, bool has_cls, double scale, int64_t comp, const Tensor& o_res) {
+  const int64_t D = check_packed(qkv, rope, heads, n_pos), B = qkv.size(0), N = qkv.size(1);
+  TORCH_CHECK_VALUE(out.dim() == 3 && out.size(0) == B && out.size(1) == N && out.size(2) == heads * D &&
+                        dout.sizes() == out.sizes(),
+                    "farope: dO and O must be [B, N, heads * head_dim]");
+  TORCH_CHECK(dout.device() == qkv.device() && out.device() == qkv.device() && lse.device() == qkv.device() &&
+                  o_res.device() == qkv.device(),
+              "farope: dO, O, LSE and O_res must be on qkv's device");
+  const Tensor g = dout.scalar_type() == qkv.scalar_type() ? dout : dout.to(qkv.scalar_type());
+  TORCH_CHECK_TYPE(out.scalar_type() == qkv.scalar_type(), "farope: O must have qkv's dtype; got ", dtype_str(out));
+  TORCH_CHECK_VALUE(lse.scalar_type() == at::kFloat && lse.dim() == 3 && lse.size(0) == B && lse.size(1) == heads &&
+                        lse.size(2) == N && lse.is_contiguous(),
+                    "farope: LSE must be contiguous fp32 [B, H, N]");
+  TORCH_CHECK_VALUE(!o_res.numel() || (o_res.dim() == 4 && o_res.numel() == out.numel() && o_res.size(1) == heads &&
+                                       o_res.scalar_type() == qkv.scalar_type() && o_res.is_contiguous()),
+                    "farope: O_res must be contiguous [B, H, N, D] of qkv's dtype, or empty");
+  const c10::DeviceGuard guard(qkv.device());
+  const farope_attn_desc desc = make_desc(B, heads, N, D, qkv.scalar_type(), n_pos, has_cls, scale, comp);
+  const Tensor dqkv = at::empty({B, N, 3 * heads * D}, qkv.options());
+  const Tensor ws = workspace(qkv, farope_attn_bwd_workspace_elems(&desc));
+  const Heads q(qkv, 0, heads, D), k(qkv, 1, heads, D), v(qkv, 2, heads, D), o(out, 0, heads, D), d(g, 0, heads, D);
+  const Heads dq(dqkv, 0, heads, D), dk(dqkv, 1, heads, D), dv(dqkv, 2, heads, D);
+  check_rc(farope_attn_bwd(&desc, q.ptr, q.st, k.ptr, k.st, v.ptr, v.st, o.ptr, o.st, data(o_res), d.ptr, d.st,
+                           lse.data_ptr<float>(), floats(rope), (size_t)rope.numel(), dq.ptr, dq.st, dk.ptr, dk.st, dv.ptr,
+                           dv.st, floats(ws), stream_of(qkv)),
+           "farope_attn_bwd");
+  return dqkv;
 }
 
 // ---------------------------------------------------------------------------
@@ -232,14 +304,90 @@ Three attn_bwd_autograd(const Tensor& dout, const Tensor& q, const Tensor& k, co
   return bwd_op().call(dout, q, k, v, o, lse, rope, n_pos, has_cls, scale, comp, o_res);
 }
 
+using QkvFwdSig = Three(const Tensor&, const Tensor&, c10::SymInt, c10::SymInt, bool, double, c10::SymInt);
+using QkvBwdSig = Tensor(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, c10::SymInt, c10::SymInt,
+                         bool, double, c10::SymInt, const Tensor&);
+const c10::TypedOperatorHandle<QkvFwdSig>& qkv_fwd_op() {
+  static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("farope::attn_qkv_fwd", "").typed<QkvFwdSig>();
+  return op;
+}
+const c10::TypedOperatorHandle<QkvBwdSig>& qkv_bwd_op() {
+  static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("farope::attn_qkv_bwd", "").typed<QkvBwdSig>();
+  return op;
+}
+
+struct QkvFwdNode : torch::autograd::Function<QkvFwdNode> {
+  static variable_list forward(torch::autograd::AutogradContext* ctx, const Tensor& qkv, const Tensor& rope, c10::SymInt heads,
+                               c10::SymInt n_pos, bool has_cls, double scale, c10::SymInt comp) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Three r = qkv_fwd_op().call(qkv, rope, heads, n_pos, has_cls, scale, comp);
+    const auto& [o, lse, o_res] = r;
+    ctx->mark_non_differentiable({lse, o_res});
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({qkv, o, lse, rope, o_res});
+    ctx->saved_data["heads"] = heads;
+    ctx->saved_data["n_pos"] = n_pos;
+    ctx->saved_data["has_cls"] = has_cls;
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["comp"] = comp;
+    return list3(r);
+  }
+  static variable_list backward(torch::autograd::AutogradContext* ctx, variable_list grads) {
+    variable_list out(7);
+    if (!grads[0].defined()) return out;
+    const variable_list s = ctx->get_saved_variables();
+    out[0] = qkv_bwd_op().call(grads[0], s[0], s[1], s[2], s[3], ctx->saved_data["heads"].toSymInt(),
+                               ctx->saved_data["n_pos"].toSymInt(), ctx->saved_data["has_cls"].toBool(),
+                               ctx->saved_data["scale"].toDouble(), ctx->saved_data["comp"].toSymInt(), s[4]);
+    return out;
+  }
+};
+
+struct QkvBwdNode : torch::autograd::Function<QkvBwdNode> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& dout, const Tensor& qkv, const Tensor& o,
+                        const Tensor& lse, const Tensor& rope, c10::SymInt heads, c10::SymInt n_pos, bool has_cls, double scale,
+                        c10::SymInt comp, const Tensor& o_res) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return qkv_bwd_op().call(dout, qkv, o, lse, rope, heads, n_pos, has_cls, scale, comp, o_res);
+  }
+  static variable_list backward(torch::autograd::AutogradContext*, variable_list) {
+    TORCH_CHECK(false,
+                "Trying to backward through farope.attn_qkv_bwd.default but no autograd formula was registered "
+                "(the attention's gradients are not differentiable again).");
+  }
+};
+
+Three attn_qkv_fwd_autograd(const Tensor& qkv, const Tensor& rope, c10::SymInt heads, c10::SymInt n_pos, bool has_cls,
+                            double scale, c10::SymInt comp) {
+  if (at::GradMode::is_enabled() && any_requires_grad({&qkv, &rope})) {
+    const variable_list r = QkvFwdNode::apply(qkv, rope, heads, n_pos, has_cls, scale, comp);
+    return {r[0], r[1], r[2]};
+  }
+  at::AutoDispatchBelowADInplaceOrView below;
+  return qkv_fwd_op().call(qkv, rope, heads, n_pos, has_cls, scale, comp);
+}
+
+Tensor attn_qkv_bwd_autograd(const Tensor& dout, const Tensor& qkv, const Tensor& o, const Tensor& lse, const Tensor& rope,
+                             c10::SymInt heads, c10::SymInt n_pos, bool has_cls, double scale, c10::SymInt comp,
+                             const Tensor& o_res) {
+  if (at::GradMode::is_enabled() && any_requires_grad({&dout, &qkv, &o, &lse, &rope, &o_res}))
+    return QkvBwdNode::apply(dout, qkv, o, lse, rope, heads, n_pos, has_cls, scale, comp, o_res);
+  at::AutoDispatchBelowADInplaceOrView below;
+  return qkv_bwd_op().call(dout, qkv, o, lse, rope, heads, n_pos, has_cls, scale, comp, o_res);
+}
+
 }  // namespace
 
 TORCH_LIBRARY_IMPL(farope, CUDA, m) {
   m.impl("attn_fwd", attn_fwd);
   m.impl("attn_bwd", attn_bwd);
+  m.impl("attn_qkv_fwd", attn_qkv_fwd);
+  m.impl("attn_qkv_bwd", attn_qkv_bwd);
 }
 
 TORCH_LIBRARY_IMPL(farope, AutogradCUDA, m) {
   m.impl("attn_fwd", attn_fwd_autograd);
   m.impl("attn_bwd", attn_bwd_autograd);
+  m.impl("attn_qkv_fwd", attn_qkv_fwd_autograd);
+  m.impl("attn_qkv_bwd", attn_qkv_bwd_autograd);
 }
