@@ -320,7 +320,7 @@ DsWs ds_ws(const farope_attn_desc* d) {
 bool stream_shape(const farope_attn_desc* d) {
   if (d->io_dtype == FAROPE_F32 || d->io_dtype != d->compute_dtype) return false;
   if (d->head_dim != 64 && d->head_dim != 32) return false;
-  return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kStreamTileRows) <= INT32_MAX;
+  return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kStreamTileRows / 2) <= INT32_MAX;
 }
 // Forward: planes past the 256 rows whose table fwd_kernel keeps in LDS.
 // Measured (us, fwd_kernel / streamed, the K-hat pass included): D 64, N 577,
@@ -641,8 +641,8 @@ int farope_tile_config(const farope_attn_desc* desc, int32_t which, int32_t out[
     out[3] = fwd_threads(D);
   } else if (bwd_stream(desc)) {
     out[0] = BWD_STREAM;
-    out[1] = kStreamTileRows;
-    out[2] = cdiv(N, kStreamTileRows);
+    out[1] = stream_rows(desc->batch * desc->heads, N, D, true);
+    out[2] = cdiv(N, out[1]);
     out[3] = kStreamThreads;
   } else {
     const bool fu = bwd_fused(desc);

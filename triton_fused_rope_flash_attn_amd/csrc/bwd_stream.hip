@@ -26,18 +26,17 @@
 namespace farope {
 
 // ---------------------------------------------------------------------------
-// dQ of 128-query tiles.  Wave w owns queries 32w .. 32w+31 (two 16-query
-// subtiles).  S^T = K-hat Q-hat^T and dP^T = V dO^T per 32-key block, keys in
+// dQ of 128-query tiles (64 with QT = 1).  Wave w owns QT 16-query subtiles.  S^T = K-hat Q-hat^T and dP^T = V dO^T per 32-key block, keys in
 // natural order: output row 4lg + i of half h is key 16h + 4lg + i, which is
 // k-slot 4h + i of the transposed reads of dQ-hat^T += K-hat^T dS^T.  Keys
 // >= N have zero K-hat and V rows: P is clamped to [0, 1] and their dS meets
 // zero rows.
 // ---------------------------------------------------------------------------
-template <typename S, int CT, int D>
+template <typename S, int CT, int D, int QT>
 __global__ void __launch_bounds__(kStreamNW * 64, 3) stream_dq_kernel(const BwdParams p) {
   using C = Comp<CT>;
   using Frag = typename C::Frag;
-  constexpr int KS = D / 32, DT = D / 16, QT = 2, SR = kStageRows;
+  constexpr int KS = D / 32, DT = D / 16, SR = kStageRows;
   __shared__ __attribute__((aligned(16))) S sK0[SR * D], sK1[SR * D], sV0[SR * D], sV1[SR * D];
 
   const int N = p.N;
@@ -60,7 +59,7 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) stream_dq_kernel(const BwdP
   srcK.load(sK0, wave, 0);
   srcV.load(sV0, wave, 0);
 
-  const int row0 = qblk * kStreamTileRows + wave * 32 + lr;   // subtile t: + 16 t
+  const int row0 = (qblk * kStreamNW + wave) * 16 * QT + lr;   // subtile t: + 16 t
   Frag qf[QT][KS], gf[QT][KS];
   f32x4 nl4[QT], nd4[QT];
   {
@@ -227,16 +226,15 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) stream_dq_kernel(const BwdP
 }
 
 // ---------------------------------------------------------------------------
-// dK / dV of 128-key tiles.  Wave w owns keys 32w .. 32w+31 (two 16-key
-// subtiles): K-hat and V rows are B operands in registers, dK-hat and dV
+// dK / dV of 128-key tiles (64 with KT = 1).  Wave w owns KT 16-key subtiles: K-hat and V rows are B operands in registers, dK-hat and dV
 // accumulate in registers.  Queries >= N have zero Q-hat and dO rows and
 // -LSE2 = -delta = 0 (reads past the range), so they add nothing.
 // ---------------------------------------------------------------------------
-template <typename S, int CT, int D>
+template <typename S, int CT, int D, int KT>
 __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const BwdParams p) {
   using C = Comp<CT>;
   using Frag = typename C::Frag;
-  constexpr int KS = D / 32, DT = D / 16, KT = 2, SR = kStageRows;
+  constexpr int KS = D / 32, DT = D / 16, SR = kStageRows;
   __shared__ __attribute__((aligned(16))) S sQ0[SR * D], sQ1[SR * D], sG0[SR * D], sG1[SR * D];
   __shared__ __attribute__((aligned(16))) float sL0[SR], sL1[SR], sD0[SR], sD1[SR];
 
@@ -266,7 +264,7 @@ __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const Bw
   };
   load(0, sQ0, sG0, sL0, sD0);
 
-  const int row0 = kblk * kStreamTileRows + wave * 32 + lr;   // subtile u: + 16 u
+  const int row0 = (kblk * kStreamNW + wave) * 16 * KT + lr;   // subtile u: + 16 u
   Frag kf[KT][KS], vf[KT][KS];
   {
     const auto rK = make_rsrc(static_cast<const S*>(p.khat) + prow * D, (unsigned)(N * D * 2));
@@ -413,12 +411,16 @@ static hipError_t stream_launch(const BwdParams& p0, hipStream_t st) {
   hipError_t e = launch_stream_khat(KhatParams{p.k, p.khat, {p.sk[0], p.sk[1], p.sk[2]}, p.rope, planes, p.H, p.N,
                                                p.has_cls, p.scale_log2}, CT, D, st);
   if (e != hipSuccess) return e;
-  p.n_blk = (p.N + kStreamTileRows - 1) / kStreamTileRows;
+  const int rows = stream_rows(planes, p.N, D, true);
+  const bool half = rows < kStreamTileRows;
+  p.n_blk = (p.N + rows - 1) / rows;
   p.n_wg = planes * p.n_blk;
-  hipLaunchKernelGGL((stream_dq_kernel<S, CT, D>), dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
+  auto dq = half ? stream_dq_kernel<S, CT, D, 1> : stream_dq_kernel<S, CT, D, 2>;
+  auto dkdv = half ? stream_dkdv_kernel<S, CT, D, 1> : stream_dkdv_kernel<S, CT, D, 2>;
+  hipLaunchKernelGGL(dq, dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((stream_dkdv_kernel<S, CT, D>), dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
+  hipLaunchKernelGGL(dkdv, dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
   return hipGetLastError();
 }
 

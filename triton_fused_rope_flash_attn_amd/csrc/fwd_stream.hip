@@ -14,8 +14,8 @@
 // Bound by the softmax VALU (16 exponentials, maxima and row-sum adds per lane
 // and 32 x 32 block against 16 MFMAs).  Measured against fwd_kernel (one 8-wave
 // workgroup per CU, 256-row tiles; us): D 64, N 577, 384 planes 89 -> 59 (K-hat
-// pass 11); N 4096, 48 planes 285 -> 211; N 1025, 64 planes 46 -> 39; D 32, N
-// 3970, 10 planes 81 -> 56.  Two or four workgroups per CU: within 1%.
+// pass 11); N 4096, 48 planes 285 -> 207; N 1025, 64 planes 46 -> 38; D 32, N
+// 3970, 10 planes 81 -> 44.  Two or four workgroups per CU: within 1%.
 #include <type_traits>
 
 #include "common.h"
@@ -49,8 +49,8 @@ __global__ void __launch_bounds__(256) stream_khat_kernel(const KhatParams p, in
 }
 
 // ---------------------------------------------------------------------------
-// O and LSE of 128-query tiles.  Wave w owns queries 32w .. 32w+31 (two
-// 16-query subtiles); logits are computed transposed, S^T = K-hat Q-hat^T, per
+// O and LSE of 128-query tiles (64 with QT = 1).  Wave w owns QT 16-query
+// subtiles; logits are computed transposed, S^T = K-hat Q-hat^T, per
 // 32-key block with keys in natural order: output row 4lg + i of half h is key
 // 16h + 4lg + i, which is k-slot 4h + i of the transposed V reads of
 // O^T += V^T P^T, so P never leaves registers.  The accumulators start at
@@ -59,11 +59,11 @@ __global__ void __launch_bounds__(256) stream_khat_kernel(const KhatParams p, in
 // ---------------------------------------------------------------------------
 constexpr float kStreamSlack = 8.0f;   // log2 units: P <= 2^8 between rescales
 
-template <typename S, int CT, int D>
+template <typename S, int CT, int D, int QT>
 __global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const FwdParams p, const S* __restrict__ khat) {
   using C = Comp<CT>;
   using Frag = typename C::Frag;
-  constexpr int KS = D / 32, DT = D / 16, QT = 2, SR = kStageRows;
+  constexpr int KS = D / 32, DT = D / 16, SR = kStageRows;
   __shared__ __attribute__((aligned(16))) S sK0[SR * D], sK1[SR * D], sV0[SR * D], sV1[SR * D];
 
   const int N = p.N;
@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const Fwd
   srcK.load(sK0, wave, 0);
   srcV.load(sV0, wave, 0);
 
-  const int row0 = qblk * kStreamTileRows + wave * 32 + lr;   // subtile t: + 16 t
+  const int row0 = (qblk * kStreamNW + wave) * 16 * QT + lr;   // subtile t: + 16 t
   Frag qf[QT][KS];
   {
     const auto rQ = rsrc(p.q, p.sq);
@@ -135,34 +135,45 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const Fwd
 #pragma unroll
   for (int d = 0; d < DT; ++d) to[d] = swz<D>(4 * lg + (lr >> 2), 16 * d + 4 * (lr & 3));
 
-  using Acc = f32x4[QT][2];
-  auto logits = [&](const S* __restrict__ k, Acc& sacc) __attribute__((always_inline)) {
+  // The stage's two 32-key blocks: both logit products, one test of the running
+  // max, then each block's probabilities and O product.  Keys at lim or beyond
+  // (counted from this lane's first; tail: there are some) get probability 0.
+  using Acc = f32x4[2][QT][2];
+  auto blocks = [&](const S* __restrict__ k, const S* __restrict__ v, bool tail, int lim) __attribute__((always_inline)) {
+    Acc sacc;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const Frag a = C::lds(k + ao[s] + 16 * h * D);
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int t = 0; t < QT; ++t) sacc[t][h] = C::mma(a, qf[t][s], s == 0 ? nm4[t] : sacc[t][h]);
-      }
-  };
-  // Softmax of one block and its O product.  Keys at lim or beyond (counted
-  // from this lane's first; tail: there are some) get probability 0.
-  auto block = [&](const S* __restrict__ v, Acc& sacc, bool tail, int lim) __attribute__((always_inline)) {
+        for (int h = 0; h < 2; ++h) {
+          const Frag a = C::lds(k + ao[s] + (32 * j + 16 * h) * D);
+#pragma unroll
+          for (int t = 0; t < QT; ++t) sacc[j][t][h] = C::mma(a, qf[t][s], s == 0 ? nm4[t] : sacc[j][t][h]);
+        }
     if (tail) {   // uniform; the plane's last stage
 #pragma unroll
-      for (int t = 0; t < QT; ++t)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int t = 0; t < QT; ++t)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) sacc[t][h][i] = 16 * h + i < lim ? sacc[t][h][i] : -INFINITY;
+          for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sacc[j][t][h][i] = 32 * j + 16 * h + i < lim ? sacc[j][t][h][i] : -INFINITY;
     }
-    float mx[QT];
+    float mx[QT], mxx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
-      mx[t] = fmaxf(fmaxf(fmaxf(sacc[t][0][0], sacc[t][0][1]), fmaxf(sacc[t][0][2], sacc[t][0][3])),
-                    fmaxf(fmaxf(sacc[t][1][0], sacc[t][1][1]), fmaxf(sacc[t][1][2], sacc[t][1][3])));
-    if (__any(fmaxf(mx[0], mx[1]) > thr)) {
+    for (int t = 0; t < QT; ++t) {
+      float y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 x = sacc[j >> 1][t][j & 1];
+        y[j] = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+      }
+      mx[t] = fmaxf(fmaxf(y[0], y[1]), fmaxf(y[2], y[3]));
+      mxx = fmaxf(mxx, mx[t]);
+    }
+    if (__any(mxx > thr)) {
       thr = kStreamSlack;
 #pragma unroll
       for (int t = 0; t < QT; ++t) {
@@ -174,28 +185,31 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const Fwd
 #pragma unroll
         for (int d = 0; d < DT; ++d) acc[t][d] *= alpha;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) sacc[t][h] += sh;
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) sacc[j][t][h] += sh;
         nm4[t] = f32x4{-mnew, -mnew, -mnew, -mnew};
       }
     }
-    Frag pf[QT];
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-      float pv[8];
+    for (int j = 0; j < 2; ++j) {
+      Frag pf[QT];
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
+      for (int t = 0; t < QT; ++t) {
+        float x[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          pv[4 * h + i] = fast_exp2(sacc[t][h][i]);
-          l_run[t] += pv[4 * h + i];
-        }
-      pf[t] = C::make(pv);
-    }
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int d = 0; d < DT; ++d) {
-      const Frag a = C::tr(v + to[d], v + to[d] + 16 * D);
+          for (int i = 0; i < 4; ++i) x[4 * h + i] = fast_exp2(sacc[j][t][h][i]);
+        l_run[t] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+        pf[t] = C::make(x);
+      }
 #pragma unroll
-      for (int t = 0; t < QT; ++t) acc[t][d] = C::mma(a, pf[t], acc[t][d]);
+      for (int d = 0; d < DT; ++d) {
+        const Frag a = C::tr(v + to[d] + 32 * j * D, v + to[d] + (32 * j + 16) * D);
+#pragma unroll
+        for (int t = 0; t < QT; ++t) acc[t][d] = C::mma(a, pf[t], acc[t][d]);
+      }
     }
   };
   auto stage = [&](int st, const S* __restrict__ k, const S* __restrict__ v, S* __restrict__ kn, S* __restrict__ vn)
@@ -209,11 +223,7 @@ __global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const Fwd
       const int left = N - st * SR;   // keys of this stage (uniform)
       const bool tail = left < SR;
       const int lim = left - 4 * lg;
-      Acc sacc;
-      logits(k, sacc);
-      block(v, sacc, tail, lim);
-      logits(k + 32 * D, sacc);
-      block(v + 32 * D, sacc, tail, lim - 32);
+      blocks(k, v, tail, lim);
     }
   };
   int st = 0;
@@ -275,9 +285,12 @@ hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st
 template <typename S, int CT, int D>
 static hipError_t fwd_stream_launch(const FwdParams& p0, const void* khat, hipStream_t st) {
   FwdParams p = p0;
-  p.n_blk = (p.N + kStreamTileRows - 1) / kStreamTileRows;
-  p.n_wg = p.B * p.H * p.n_blk;
-  hipLaunchKernelGGL((fwd_stream_kernel<S, CT, D>), dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p, static_cast<const S*>(khat));
+  const int planes = p.B * p.H;
+  const int rows = stream_rows(planes, p.N, D, false);
+  p.n_blk = (p.N + rows - 1) / rows;
+  p.n_wg = planes * p.n_blk;
+  auto kern = rows < kStreamTileRows ? fwd_stream_kernel<S, CT, D, 1> : fwd_stream_kernel<S, CT, D, 2>;
+  hipLaunchKernelGGL(kern, dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p, static_cast<const S*>(khat));
   return hipGetLastError();
 }
 hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st) {

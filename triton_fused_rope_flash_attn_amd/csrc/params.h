@@ -130,8 +130,20 @@ hipError_t launch_bwd_ds_dq(const BwdParams& p, int io, hipStream_t st);
 
 // Streamed-tile backward (bwd_stream.hip): p.delta, p.row_stat (-LSE2 rows),
 // p.qhat_f and p.khat are its workspace.
-constexpr int kStreamTileRows = 128;   // rows per workgroup (forward, dQ, dK/dV)
+constexpr int kStreamTileRows = 128;   // rows per workgroup (forward, dQ, dK/dV) of large calls
 constexpr int kStreamThreads = 256;
+// Rows per workgroup of a call: 64 (one 16-row subtile per wave) while its
+// 128-row tiles are too few for the workgroups that fit on the chip at once.
+// Measured (us, 128 / 64 rows; the call's 128-row tiles in brackets), forward, D
+// 64: [33] 21.2 / 15.5, [60] 13.6 / 10.6, [108] 18.5 / 13.9, [240] 15.3 / 14.3, [384]
+// 44.3 / 39.8, [480] 23.7 / 23.8, [960] 36.4 / 37.6; D 32: [320] 54.7 / 44.2, [640]
+// 18.5 / 16.9.  Backward, D 64: [33] 51.6 / 37.1, [60] 31.0 / 22.7, [240] 34.2 / 31.4,
+// [384] 108 / 102, [480] 48.4 / 50.0, [960] 81 / 87; D 32: [320] 133 / 119, [640] 39.2 /
+// 38.6.  (The backward's results are the same bit for bit.)
+inline int stream_rows(int planes, int N, int D, bool backward) {
+  const int64_t tiles = (int64_t)planes * ((N + kStreamTileRows - 1) / kStreamTileRows);
+  return tiles <= (D == 32 ? 768 : backward ? 400 : 512) ? kStreamTileRows / 2 : kStreamTileRows;
+}
 // K-hat * c2 rows [planes][N][D] of 16-bit K (any vector-access strides), in
 // the compute type: what both passes stream.
 struct KhatParams {
