@@ -255,7 +255,8 @@ int farope_attn_bwd_noalloc(const farope_attn_desc* desc,
  * 1 = one wave per (b, h) plane for 193 <= N <= 208 at head_dim 64 with
  * 16-bit tensors, assuming vector access (the streamed query tiles of
  * farope_attn_fwd_ws and, in either pass, the 64-row short-plane kernels that
- * take calls of few or short planes at head_dim 32 and 64 are not reported); bwd: 0 fused, 1 split, 2 split with
+ * take calls of few or short planes at head_dim 32 and 64 are not reported, nor
+ * the 128-row items of forward calls of few planes at head_dim 128); bwd: 0 fused, 1 split, 2 split with
  * the key-tile kernel, 3 key tiles that store dS and dQ as one GEMM over it,
  * 4 streamed tiles, assuming vector access), out[1] = query (fwd) or key (bwd) rows per work item,
  * out[2] = work items per (b, h) plane, out[3] = threads per workgroup.  When 1 to 8 rows are left past out[1] * out[2] (N = 1025 with

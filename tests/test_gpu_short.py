@@ -7,7 +7,7 @@ import torch
 from oracle import torch_ref
 from tests.cases import ROPE_BASE, TOL_MEAN
 from tests.test_gpu_parity import _compare
-from triton_fused_rope_flash_attn_amd import CosSinTable, _lib
+from triton_fused_rope_flash_attn_amd import CosSinTable, _lib, sdpa_triton_fa_rope
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -63,3 +63,24 @@ def test_short_planes(side, has_cls, D, io):
     # a logit of size s is off by about 2^-8 s (bf16 operands)
     assert (got[1] - lse).abs().max().item() < (1e-4 if io == "fp32" else 2e-2)
     assert all(torch.equal(a, b) for a, b in zip(got, run()))
+
+
+@pytest.mark.parametrize("side,has_cls,dt,B", [(11, False, "bf16", 2), (14, True, "bf16", 2), (16, True, "bf16", 2),
+                                               (16, False, "fp16", 2), (19, False, "fp16", 2), (32, True, "bf16", 1),
+                                               (14, True, "bf16", 44)])   # 264 items of 128 rows: the 256-row ones
+def test_wide_planes_of_small_calls(side, has_cls, dt, B):
+    """head_dim 128 forward: 128-row items (one subtile per wave) while they fit one
+    per CU.  Rows past the last item (N = 257: the folded row), planes shorter
+    than an item, and a call past the limit."""
+    H, D = 3, 128
+    N = side * side + int(has_cls)
+    dt = DT[dt]
+    print(f"wide planes N={N} B={B} {dt}", flush=True)
+    g = torch.Generator().manual_seed(62)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    q, k, v, do = (torch.randn(B, H, N, D, generator=g).to(dt).to(DEV) for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    o = sdpa_triton_fa_rope(*leaves, table, H_img=side, has_cls=has_cls)
+    got = (o.detach(), *torch.autograd.grad(o, leaves, do))
+    ref = torch_ref.forward_backward(*(t.detach().float() for t in (q, k, v)), do.float(), *table.tables(), has_cls)
+    _compare(f"wide-N{N}-B{B}", got, ref, out_dtype=dt)

@@ -569,7 +569,7 @@ int fwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
     FAROPE_TRY(launch_rc(launch_stream_khat(kp, desc->compute_dtype, desc->head_dim, st)));
     return launch_rc(launch_fwd_stream(p, ws, desc->io_dtype, desc->head_dim, st));
   }
-  const int rows = fwd_block_rows(desc->head_dim, desc->io_dtype, desc->compute_dtype);
+  const int rows = fwd_call_rows(desc->head_dim, desc->io_dtype, desc->compute_dtype, p.B * p.H, p.N);
   const int tail = tail_of(p.B * p.H, p.N, rows);
   p.n_blk = main_blocks(p.B * p.H, p.N, rows);
   p.n_items = p.B * p.H * p.n_blk;

@@ -1354,6 +1354,8 @@ template <> struct FwdShape<128> { static constexpr int NW = 8, QT = 1, KC = 64,
 // 512 registers (VGPRs plus AGPRs): the O accumulators alone are 64 per wave.
 template <> struct FwdShape<256> { static constexpr int NW = 4, QT = 1, KC = 32, TABROWS = 0; };
 
+constexpr int kFwdCus = 256;   // CUs of the chip
+
 // Query subtiles per wave at D = 128: two with 16-bit tensors and 16-bit
 // compute, so that every staged K-hat chunk (rotated and converted once per
 // item) serves twice the queries; their Q rows
@@ -1369,6 +1371,17 @@ template <int D> static int fwd_rows_of(int io, int ct) {
 int fwd_block_rows(int D, int io, int ct) {
   return D == 32 ? fwd_rows_of<32>(io, ct) : D == 64 ? fwd_rows_of<64>(io, ct)
          : D == 128 ? fwd_rows_of<128>(io, ct) : fwd_rows_of<256>(io, ct);
+}
+// Query rows per item of a call: at D = 128 one subtile per wave (128 rows)
+// while those items still fit the chip at one workgroup per CU; two subtiles
+// (256 rows) halve the staging per query once every CU is busy.  Measured (us,
+// 256 / 128 rows; 128-row items in brackets): bf16 [24] 20.4 / 15.2, [108] 58.5 /
+// 45.0, [192] 21.5 / 16.3, [240] 36.8 / 27.1, [432] 60.4 / 79.9, [768] 326 / 348;
+// fp16 compute [96] 25.2 / 20.8, [384] 18.1 / 26.2.  Bit-identical (bf16).
+int fwd_call_rows(int D, int io, int ct, int planes, int N) {
+  const int rows = fwd_block_rows(D, io, ct), one = FwdShape<128>::NW * 16;
+  if (D == 128 && rows > one && (int64_t)planes * ((N + one - 1) / one) <= kFwdCus) return one;
+  return rows;
 }
 int fwd_threads(int D) {
   return 64 * (D == 32    ? FwdShape<32>::NW
@@ -1393,6 +1406,10 @@ static hipError_t fwd_launch(const FwdParams& p0, hipStream_t st) {
                          : fwd_kernel<IO, CT, D, SH::NW, QT, SH::KC, TR, false, FS>)
                   : (vec ? fwd_kernel<IO, CT, D, SH::NW, QT, SH::KC, 0, true, FS>
                          : fwd_kernel<IO, CT, D, SH::NW, QT, SH::KC, 0, false, FS>);
+  if constexpr (D == 128 && QT == 2) {
+    if (fwd_call_rows(D, DT_F16, CT, p.B * p.H, p.N) == SH::NW * 16)   // (16-bit tensors)
+      kern = vec ? fwd_kernel<IO, CT, D, SH::NW, 1, SH::KC, 0, true, FS> : fwd_kernel<IO, CT, D, SH::NW, 1, SH::KC, 0, false, FS>;
+  }
   const int grid = persistent_grid(reinterpret_cast<const void*>(kern), SH::NW * 64, p.n_items);
   if (grid <= 0) return hipErrorInvalidConfiguration;
   p.n_wg = grid;

@@ -196,6 +196,7 @@ int persistent_grid(const void* kernel, int block_threads, int items, size_t dyn
 
 // Rows of q (fwd, dq) or kv (dk/dv) one work item / workgroup covers.
 int fwd_block_rows(int D, int io, int ct);
+int fwd_call_rows(int D, int io, int ct, int planes, int N);   // of a call: fwd_block_rows, or 128 of 256
 int fwd_threads(int D);
 int bwd_dq_block_rows(int D, int ct);
 int bwd_dkdv_block_rows(int D, int ct);
