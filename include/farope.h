@@ -130,9 +130,10 @@ size_t farope_attn_residual_elems(const farope_attn_desc* desc);
  * per key tile; the key tiles' fp16 K-hat rows; and their fp16 dS^T rows
  * (pitch seq_len rounded up to 64), which the dQ GEMM reads instead of
  * recomputing the logits.  At the streamed shapes (16-bit tensors computed in
- * their own type, head_dim 64 and seq_len > 257 or head_dim 32 and seq_len >
- * 256; each part from a 256-byte boundary): -delta and -LSE * log2(e) rows, then the rotated Q rows and the
- * rotated, scaled K rows in 16 bits.  0 on an invalid descriptor.
+ * their own type, head_dim 64, or 128 in fp16, and seq_len > 257, or head_dim
+ * 32 and seq_len > 256; each part from a 256-byte boundary): -delta and
+ * -LSE * log2(e) rows, then the rotated Q rows and the rotated, scaled K rows in
+ * 16 bits.  0 on an invalid descriptor.
  */
 size_t farope_attn_bwd_workspace_elems(const farope_attn_desc* desc);
 
@@ -153,10 +154,10 @@ int farope_attn_fwd(const farope_attn_desc* desc,
 /*
  * farope_attn_fwd with a caller workspace of farope_attn_fwd_workspace_elems(desc)
  * fp32 elements (16-byte aligned; NULL: as farope_attn_fwd).  Where that is not
- * 0 (16-bit tensors computed in their own type, head_dim 32 or 64, seq_len >
- * 256) and every tensor allows vector access, the rotated K rows are written
- * there once and streamed by every query tile; otherwise it is not used.  No
- * counterpart in the reference.
+ * 0 (16-bit tensors computed in their own type, head_dim 32 or 64, or 128 in
+ * fp16, and seq_len > 256) and every tensor allows vector access, the rotated
+ * K rows are written there once and streamed by every query tile; otherwise it
+ * is not used.  No counterpart in the reference.
  */
 size_t farope_attn_fwd_workspace_elems(const farope_attn_desc* desc);
 int farope_attn_fwd_ws(const farope_attn_desc* desc,

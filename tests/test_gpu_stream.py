@@ -54,6 +54,7 @@ def _views(B, H, N, D, dt, gen, pad=0):
     (17, False, 64, "bf16"), (17, True, 64, "fp16"), (18, False, 64, "bf16"), (19, False, 64, "bf16"),
     (20, False, 64, "fp16"), (24, True, 64, "bf16"), (32, False, 64, "bf16"), (32, True, 64, "bf16"),
     (16, True, 32, "bf16"), (17, True, 32, "fp16"), (24, False, 32, "bf16"), (31, True, 32, "bf16"),
+    (17, True, 128, "fp16"), (20, False, 128, "fp16"), (21, True, 128, "fp16"), (24, True, 128, "fp16"),
 ])
 def test_streamed_tiles(side, has_cls, D, dt, B, H):
     N = side * side + int(has_cls)
@@ -61,7 +62,7 @@ def test_streamed_tiles(side, has_cls, D, dt, B, H):
         pytest.skip("the 128-row tiles' remainders are covered by the shorter planes")
     code = {"bf16": _lib.BF16, "fp16": _lib.F16}[dt]
     rows = _lib.tile_config(_lib.make_desc(B, H, N, D, N - int(has_cls), has_cls, code, code, 0.1), 1)[1]
-    assert rows == (64 if B == 2 else 128)
+    assert rows == (64 if B == 2 or D == 128 else 128)
     dt = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
     print(f"streamed N={N} D={D} {dt}", flush=True)
     table = CosSinTable(ROPE_BASE, side, D, device=DEV)

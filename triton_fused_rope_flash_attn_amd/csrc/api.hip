@@ -315,25 +315,30 @@ DsWs ds_ws(const farope_attn_desc* d) {
 }
 
 // The streamed tiles (fwd_stream.hip, bwd_stream.hip): 16-bit tensors computed
-// in their own type at head_dim 32 or 64.  (Vector access to every tensor is
-// checked at the call.)
+// in their own type at head_dim 32 or 64, or in fp16 at 128.  (Vector access to
+// every tensor is checked at the call.)
 bool stream_shape(const farope_attn_desc* d) {
   if (d->io_dtype == FAROPE_F32 || d->io_dtype != d->compute_dtype) return false;
-  if (d->head_dim != 64 && d->head_dim != 32) return false;
+  // (head_dim 128 with bf16 compute takes fp16 logit operands: other kernels)
+  if (d->head_dim != 64 && d->head_dim != 32 && !(d->head_dim == 128 && d->compute_dtype == FAROPE_F16)) return false;
   return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kStreamTileRows / 2) <= INT32_MAX;
 }
 // Forward: planes past the 256 rows whose table fwd_kernel keeps in LDS.
 // Measured (us, fwd_kernel / streamed, the K-hat pass included): D 64, N 577,
 // 384 planes 89 / 59; N 257, 1536 planes 90 / 78; N 256 52 / 59; N 170, 3072
-// planes 81 / 107.  D 32: N 257, 512 planes 32 / 25; N 256 15 / 20.
+// planes 81 / 107.  D 32: N 257, 512 planes 32 / 25; N 256 15 / 20.  D 128, fp16: N
+// 257, 384 planes 54 / 47; N 577 137 / 120; N 1025, 12 planes 51 / 24; N 4096, 24
+// planes 295 / 207.
 bool fwd_stream(const farope_attn_desc* d) { return stream_shape(d) && d->seq_len > kPlaneMaxN; }
-// Backward: planes past the one-pass kernel's 256 rows at head_dim 64 (it
-// stays at N = 257, whose delta-only workspace callers rely on), and past the
-// same length at head_dim 32.  Measured (us, bwd_dq_kernel + bwd_dkdv_kernel /
-// streamed): D 64, N 577, 384 planes 264 / 165; N 4096, 48 planes 795 / 618;
-// N 324, 24 planes 42 / 24.  D 32, N 257, 512 planes 71 / 46.
+// Backward: planes past the one-pass kernel's 256 rows at head_dim 64, and past
+// the same length at 32 and 128.  (Not N = 257 at 64 and 128: its workspace of
+// delta rows alone is what callers of the C ABI allocate.)  Measured (us,
+// bwd_dq_kernel + bwd_dkdv_kernel / streamed): D 64, N 577, 384 planes 264 / 165; N 4096, 48 planes 795 / 618;
+// N 324, 24 planes 42 / 24.  D 32, N 257, 512 planes 71 / 46.  D 128, fp16: N 577,
+// 384 planes 497 / 368; N 1024 1024 / 888; N 1025, 12 planes 142 / 58; N 289, 96
+// planes 69 / 42.
 bool bwd_stream(const farope_attn_desc* d) {
-  return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim == 64 ? 1 : 0);
+  return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim >= 64 ? 1 : 0);
 }
 // The short-plane kernels (short.hip): tensors in the compute type or in fp32,
 // head_dim 32 or 64, N <= 256.  (Vector access to every tensor is checked at
@@ -641,7 +646,7 @@ int farope_tile_config(const farope_attn_desc* desc, int32_t which, int32_t out[
     out[3] = fwd_threads(D);
   } else if (bwd_stream(desc)) {
     out[0] = BWD_STREAM;
-    out[1] = stream_rows(desc->batch * desc->heads, N, D, true);
+    out[1] = D == 128 ? kStreamTileRows / 2 : stream_rows(desc->batch * desc->heads, N, D, true);
     out[2] = cdiv(N, out[1]);
     out[3] = kStreamThreads;
   } else {

@@ -1,6 +1,6 @@
-// Split backward with streamed tiles: head_dim 32 or 64, 16-bit tensors
-// computed in their own type, vector access to every tensor, planes longer
-// than the one-pass kernel takes.
+// Split backward with streamed tiles: 16-bit tensors computed in their own type
+// at head_dim 32 or 64, or in fp16 at 128; vector access to every tensor, planes
+// longer than the one-pass kernel takes.
 //
 // Reference behaviour followed ("fa_rope_full .py"): delta = rowsum(dO * O)
 // (FA:325-357); dV += P^T dO, dS = P * (dP - delta), dK-hat += dS^T Q-hat
@@ -33,7 +33,7 @@ namespace farope {
 // zero rows.
 // ---------------------------------------------------------------------------
 template <typename S, int CT, int D, int QT>
-__global__ void __launch_bounds__(kStreamNW * 64, 3) stream_dq_kernel(const BwdParams p) {
+__global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) stream_dq_kernel(const BwdParams p) {
   using C = Comp<CT>;
   using Frag = typename C::Frag;
   constexpr int KS = D / 32, DT = D / 16, SR = kStageRows;
@@ -416,17 +416,23 @@ static hipError_t stream_launch(const BwdParams& p0, hipStream_t st) {
   p.n_blk = (p.N + rows - 1) / rows;
   p.n_wg = planes * p.n_blk;
   auto dq = half ? stream_dq_kernel<S, CT, D, 1> : stream_dq_kernel<S, CT, D, 2>;
-  auto dkdv = half ? stream_dkdv_kernel<S, CT, D, 1> : stream_dkdv_kernel<S, CT, D, 2>;
   hipLaunchKernelGGL(dq, dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  // (D 128: the dK / dV accumulators of two subtiles alone would take 128 registers)
+  constexpr int KTM = D == 128 ? 1 : 2;
+  const int krows = half ? kStreamTileRows / 2 : kStreamTileRows / 2 * KTM;
+  p.n_blk = (p.N + krows - 1) / krows;
+  p.n_wg = planes * p.n_blk;
+  auto dkdv = half ? stream_dkdv_kernel<S, CT, D, 1> : stream_dkdv_kernel<S, CT, D, KTM>;
   hipLaunchKernelGGL(dkdv, dim3(p.n_wg), dim3(kStreamNW * 64), 0, st, p);
   return hipGetLastError();
 }
 
 hipError_t launch_bwd_stream(const BwdParams& p, int io, int D, hipStream_t st) {
   if (io == DT_BF16) return D == 64 ? stream_launch<bf16, DT_BF16, 64>(p, st) : stream_launch<bf16, DT_BF16, 32>(p, st);
-  return D == 64 ? stream_launch<f16, DT_F16, 64>(p, st) : stream_launch<f16, DT_F16, 32>(p, st);
+  return D == 128 ? stream_launch<f16, DT_F16, 128>(p, st)
+         : D == 64 ? stream_launch<f16, DT_F16, 64>(p, st) : stream_launch<f16, DT_F16, 32>(p, st);
 }
 
 }  // namespace farope

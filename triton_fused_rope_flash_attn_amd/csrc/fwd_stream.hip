@@ -1,5 +1,5 @@
-// Forward with streamed tiles: head_dim 32 or 64, 16-bit tensors computed in
-// their own type, vector access to every tensor.
+// Forward with streamed tiles: 16-bit tensors computed in their own type at
+// head_dim 32 or 64, or in fp16 at 128; vector access to every tensor.
 //
 // Reference behaviour followed: _attn_fwd in "fa_rope_full .py" (FA:91-315):
 // rotation with the CLS row bypassing it (FA:176-202, FA:248-272), scaled
@@ -15,7 +15,8 @@
 // and 32 x 32 block against 16 MFMAs).  Measured against fwd_kernel (one 8-wave
 // workgroup per CU, 256-row tiles; us): D 64, N 577, 384 planes 89 -> 59 (K-hat
 // pass 11); N 4096, 48 planes 285 -> 207; N 1025, 64 planes 46 -> 38; D 32, N
-// 3970, 10 planes 81 -> 44.  Two or four workgroups per CU: within 1%.
+// 3970, 10 planes 81 -> 44; D 128, fp16, N 577, 384 planes
+// 137 -> 120.  Two or four workgroups per CU (D 32 and 64): within 1%.
 #include <type_traits>
 
 #include "common.h"
@@ -60,7 +61,7 @@ __global__ void __launch_bounds__(256) stream_khat_kernel(const KhatParams p, in
 constexpr float kStreamSlack = 8.0f;   // log2 units: P <= 2^8 between rescales
 
 template <typename S, int CT, int D, int QT>
-__global__ void __launch_bounds__(kStreamNW * 64, 3) fwd_stream_kernel(const FwdParams p, const S* __restrict__ khat) {
+__global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) fwd_stream_kernel(const FwdParams p, const S* __restrict__ khat) {
   using C = Comp<CT>;
   using Frag = typename C::Frag;
   constexpr int KS = D / 32, DT = D / 16, SR = kStageRows;
@@ -272,10 +273,8 @@ template <typename S, int CT>
 static hipError_t khat_launch(const KhatParams& p, int D, hipStream_t st) {
   const int64_t wg = ((int64_t)p.planes * p.N * (D / 8) + 255) / 256;
   const int n_wg = (int)(wg < 8192 ? wg : 8192);
-  if (D == 64)
-    hipLaunchKernelGGL((stream_khat_kernel<S, CT, 64>), dim3(n_wg), dim3(256), 0, st, p, n_wg);
-  else
-    hipLaunchKernelGGL((stream_khat_kernel<S, CT, 32>), dim3(n_wg), dim3(256), 0, st, p, n_wg);
+  auto kern = D == 128 ? stream_khat_kernel<S, CT, 128> : D == 64 ? stream_khat_kernel<S, CT, 64> : stream_khat_kernel<S, CT, 32>;
+  hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), 0, st, p, n_wg);
   return hipGetLastError();
 }
 hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st) {
@@ -295,7 +294,8 @@ static hipError_t fwd_stream_launch(const FwdParams& p0, const void* khat, hipSt
 }
 hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st) {
   if (io == DT_BF16) return D == 64 ? fwd_stream_launch<bf16, DT_BF16, 64>(p, khat, st) : fwd_stream_launch<bf16, DT_BF16, 32>(p, khat, st);
-  return D == 64 ? fwd_stream_launch<f16, DT_F16, 64>(p, khat, st) : fwd_stream_launch<f16, DT_F16, 32>(p, khat, st);
+  return D == 128 ? fwd_stream_launch<f16, DT_F16, 128>(p, khat, st)
+         : D == 64 ? fwd_stream_launch<f16, DT_F16, 64>(p, khat, st) : fwd_stream_launch<f16, DT_F16, 32>(p, khat, st);
 }
 
 }  // namespace farope

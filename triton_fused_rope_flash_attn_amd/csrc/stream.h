@@ -15,7 +15,9 @@ constexpr int kStageRows = 64;                // streamed rows per stage
 // are XOR-swizzled per row with period 16: 16-byte reads of 16 consecutive
 // rows and transposed reads of rows 4lg + e are free of bank conflicts.
 template <int D> __device__ __forceinline__ int swz_chunk(int r) {
-  if constexpr (D == 64)
+  if constexpr (D == 128)  // (the low chunk bit stays: rows of 16 chunks cover all banks)
+    return ((r >> 1) & 7) << 1;
+  else if constexpr (D == 64)
     return ((((r >> 1) & 3) ^ ((r >> 2) & 2)) << 1) | ((r >> 3) & 1);
   else
     return (r >> 2) & 3;
