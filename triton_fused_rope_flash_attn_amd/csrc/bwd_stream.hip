@@ -26,8 +26,9 @@
 namespace farope {
 
 // ---------------------------------------------------------------------------
-// dQ of 128-query tiles (64 with QT = 1).  Wave w owns QT 16-query subtiles.  S^T = K-hat Q-hat^T and dP^T = V dO^T per 32-key block, keys in
-// natural order: output row 4lg + i of half h is key 16h + 4lg + i, which is
+// dQ of 128-query tiles (64 with QT = 1).  Wave w owns QT 16-query subtiles.
+// S^T = K-hat Q-hat^T and dP^T = V dO^T per 32-key block, keys in natural
+// order: output row 4lg + i of half h is key 16h + 4lg + i, which is
 // k-slot 4h + i of the transposed reads of dQ-hat^T += K-hat^T dS^T.  Keys
 // >= N have zero K-hat and V rows: P is clamped to [0, 1] and their dS meets
 // zero rows.
