@@ -17,6 +17,11 @@
 // barrier per stage.  Workgroups are 4 waves of 32 rows each, two (dK/dV) or
 // three (dQ) on a CU: their barriers are independent, so one workgroup's
 // MFMAs run under another's softmax and stage waits.
+//
+// Bound by instruction issue (MFMA and the softmax VALU; every operand crosses
+// HBM about once).  Measured against bwd_dq_kernel + bwd_dkdv_kernel (us): D 64,
+// N 577, 384 planes 264 -> 159; N 4096, 48 planes 795 -> 597; D 32, N 257, 512
+// planes 71 -> 43; D 128, fp16, N 577, 384 planes 497 -> 368.
 #include <type_traits>
 
 #include "common.h"
@@ -30,8 +35,11 @@ namespace farope {
 // S^T = K-hat Q-hat^T and dP^T = V dO^T per 32-key block, keys in natural
 // order: output row 4lg + i of half h is key 16h + 4lg + i, which is
 // k-slot 4h + i of the transposed reads of dQ-hat^T += K-hat^T dS^T.  Keys
-// >= N have zero K-hat and V rows: P is clamped to [0, 1] and their dS meets
-// zero rows.
+// >= N have zero K-hat and V rows: in the last stage P is clamped to [0, 1] and
+// their dS meets zero rows.  The last stage stands apart, so that the others
+// hold neither the clamp nor a test of the plane's end (us, backward, this
+// kernel and the next one so: N 4096, 48 planes 625 -> 597; N 577, 384 planes
+// 163 -> 158; N 1025, 12 planes 32.0 -> 29.9).
 // ---------------------------------------------------------------------------
 template <typename S, int CT, int D, int QT>
 __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) stream_dq_kernel(const BwdParams p) {
@@ -140,7 +148,8 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) s
         }
       }
   };
-  auto out = [&](const S* __restrict__ k, const Acc& sacc, const Acc& pacc) __attribute__((always_inline)) {
+  // clamp: the block may hold keys >= N, whose P may overflow
+  auto out = [&](auto clamp, const S* __restrict__ k, const Acc& sacc, const Acc& pacc) __attribute__((always_inline)) {
     Frag dsf[QT];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
@@ -148,8 +157,10 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) s
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          ds[4 * h + i] = __builtin_amdgcn_fmed3f(fast_exp2(sacc[t][h][i]), 0.f, 1.f) * pacc[t][h][i];
+        for (int i = 0; i < 4; ++i) {
+          const float e = fast_exp2(sacc[t][h][i]);
+          ds[4 * h + i] = (clamp.value ? __builtin_amdgcn_fmed3f(e, 0.f, 1.f) : e) * pacc[t][h][i];
+        }
       dsf[t] = C::make(ds);
     }
 #pragma unroll
@@ -159,34 +170,39 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) s
       for (int t = 0; t < QT; ++t) acc[t][d] = C::mma(a, dsf[t], acc[t][d]);
     }
   };
-  auto stage = [&](int st, const S* __restrict__ k, const S* __restrict__ v, S* __restrict__ kn, S* __restrict__ vn)
+  auto stage = [&](auto last, int st, const S* __restrict__ k, const S* __restrict__ v, S* __restrict__ kn, S* __restrict__ vn)
       __attribute__((always_inline)) {
     // every load into (k, v) has landed in every wave, and every wave is past
     // its reads of (kn, vn)
     stage_barrier();
-    if (st + 1 < ns) {
+    if (!last.value) {
       srcK.load(kn, wave, (st + 1) * SR);
       srcV.load(vn, wave, (st + 1) * SR);
     }
     if (active) {
       Acc sA, pA, sB, pB;
-      if (st * SR + 32 < N) {
+      if (!last.value || st * SR + 32 < N) {
         sp(k, v, sA, pA);
         sp(k + 32 * D, v + 32 * D, sB, pB);
-        out(k, sA, pA);
-        out(k + 32 * D, sB, pB);
+        out(last, k, sA, pA);
+        out(last, k + 32 * D, sB, pB);
       } else {
         sp(k, v, sA, pA);
-        out(k, sA, pA);
+        out(last, k, sA, pA);
       }
     }
   };
   int st = 0;
-  for (; st + 1 < ns; st += 2) {
-    stage(st, sK0, sV0, sK1, sV1);
-    stage(st + 1, sK1, sV1, sK0, sV0);
+  for (; st + 2 < ns; st += 2) {
+    stage(std::false_type{}, st, sK0, sV0, sK1, sV1);
+    stage(std::false_type{}, st + 1, sK1, sV1, sK0, sV0);
   }
-  if (st < ns) stage(st, sK0, sV0, sK1, sV1);
+  if (st + 1 < ns) {
+    stage(std::false_type{}, st, sK0, sV0, sK1, sV1);
+    stage(std::true_type{}, st + 1, sK1, sV1, sK0, sV0);
+  } else {
+    stage(std::true_type{}, st, sK0, sV0, sK1, sV1);
+  }
 
   // dQ = R^T dQ-hat * scale (K-hat carries c2); lane groups lg and lg^1 trade
   // halves so that each lane stores 8 consecutive channels; rows >= N drop
@@ -337,13 +353,13 @@ __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const Bw
       }
     }
   };
-  auto stage = [&](int st, const S* __restrict__ q, const S* __restrict__ g, const float* __restrict__ l, const float* __restrict__ dl,
+  auto stage = [&](auto last, int st, const S* __restrict__ q, const S* __restrict__ g, const float* __restrict__ l, const float* __restrict__ dl,
                    S* __restrict__ qn, S* __restrict__ gn, float* __restrict__ ln, float* __restrict__ dn) __attribute__((always_inline)) {
     stage_barrier();
-    if (st + 1 < ns) load(st + 1, qn, gn, ln, dn);
+    if (!last.value) load(st + 1, qn, gn, ln, dn);
     if (active) {
       Acc sA, pA;
-      if (st * SR + 32 < N) {
+      if (!last.value || st * SR + 32 < N) {
         Acc sB, pB;
         sp(q, g, l, dl, sA, pA);
         sp(q + 32 * D, g + 32 * D, l + 32, dl + 32, sB, pB);
@@ -356,11 +372,16 @@ __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const Bw
     }
   };
   int st = 0;
-  for (; st + 1 < ns; st += 2) {
-    stage(st, sQ0, sG0, sL0, sD0, sQ1, sG1, sL1, sD1);
-    stage(st + 1, sQ1, sG1, sL1, sD1, sQ0, sG0, sL0, sD0);
+  for (; st + 2 < ns; st += 2) {
+    stage(std::false_type{}, st, sQ0, sG0, sL0, sD0, sQ1, sG1, sL1, sD1);
+    stage(std::false_type{}, st + 1, sQ1, sG1, sL1, sD1, sQ0, sG0, sL0, sD0);
   }
-  if (st < ns) stage(st, sQ0, sG0, sL0, sD0, sQ1, sG1, sL1, sD1);
+  if (st + 1 < ns) {
+    stage(std::false_type{}, st, sQ0, sG0, sL0, sD0, sQ1, sG1, sL1, sD1);
+    stage(std::true_type{}, st + 1, sQ1, sG1, sL1, sD1, sQ0, sG0, sL0, sD0);
+  } else {
+    stage(std::true_type{}, st, sQ0, sG0, sL0, sD0, sQ1, sG1, sL1, sD1);
+  }
 
   const auto rdK = rsrc(p.dk, p.sdk), rdV = rsrc(p.dv, p.sdv);
   const auto rT = make_rsrc(p.rope, (unsigned)((N + shift) * D * 4));

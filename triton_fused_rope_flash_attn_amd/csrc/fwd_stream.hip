@@ -13,10 +13,10 @@
 //
 // Bound by the softmax VALU (16 exponentials, maxima and row-sum adds per lane
 // and 32 x 32 block against 16 MFMAs).  Measured against fwd_kernel (one 8-wave
-// workgroup per CU, 256-row tiles; us): D 64, N 577, 384 planes 89 -> 59 (K-hat
-// pass 11); N 4096, 48 planes 285 -> 207; N 1025, 64 planes 46 -> 38; D 32, N
-// 3970, 10 planes 81 -> 44; D 128, fp16, N 577, 384 planes
-// 137 -> 120.  Two or four workgroups per CU (D 32 and 64): within 1%.
+// workgroup per CU, 256-row tiles; us): D 64, N 577, 384 planes 89 -> 58 (K-hat
+// pass 11); N 4096, 48 planes 285 -> 207; N 1025, 64 planes 46 -> 37; D 32, N
+// 3970, 10 planes 81 -> 43; D 128, fp16, N 577, 384 planes 137 -> 118.  Two or
+// four workgroups per CU (D 32 and 64): within 1%.
 #include <type_traits>
 
 #include "common.h"
@@ -231,26 +231,44 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) f
       }
     }
   };
-  auto stage = [&](int st, const S* __restrict__ k, const S* __restrict__ v, S* __restrict__ kn, S* __restrict__ vn)
+  // last (a type, or a run-time value): no stage follows, keys may end in this one
+  auto stage = [&](auto last, int st, const S* __restrict__ k, const S* __restrict__ v, S* __restrict__ kn, S* __restrict__ vn)
       __attribute__((always_inline)) {
     stage_barrier();
-    if (st + 1 < ns) {
+    if (!last) {
       srcK.load(kn, wave, (st + 1) * SR);
       srcV.load(vn, wave, (st + 1) * SR);
     }
     if (active) {
       const int left = N - st * SR;   // keys of this stage (uniform)
-      const bool tail = left < SR;
+      const bool tail = !std::is_same_v<decltype(last), std::false_type> && left < SR;
       const int lim = left - 4 * lg;
       blocks(k, v, tail, lim);
     }
   };
+  // The last stage apart, so that the others hold no test of the plane's end.
+  // Measured (us, tests in every stage / apart): 12 planes of N 1025, QT 1 13.9
+  // / 13.4; D 32, N 3970, 10 planes 44.1 / 42.9; D 128, N 4096 212 / 209; but D
+  // 64, QT 2, N 577, 384 planes 58.7 / 59.4, which keeps the tests.
   int st = 0;
-  for (; st + 1 < ns; st += 2) {
-    stage(st, sK0, sV0, sK1, sV1);
-    stage(st + 1, sK1, sV1, sK0, sV0);
+  if constexpr (D == 64 && QT == 2) {
+    for (; st + 1 < ns; st += 2) {
+      stage(st + 1 >= ns, st, sK0, sV0, sK1, sV1);
+      stage(st + 2 >= ns, st + 1, sK1, sV1, sK0, sV0);
+    }
+    if (st < ns) stage(st + 1 >= ns, st, sK0, sV0, sK1, sV1);
+  } else {
+    for (; st + 2 < ns; st += 2) {
+      stage(std::false_type{}, st, sK0, sV0, sK1, sV1);
+      stage(std::false_type{}, st + 1, sK1, sV1, sK0, sV0);
+    }
+    if (st + 1 < ns) {
+      stage(std::false_type{}, st, sK0, sV0, sK1, sV1);
+      stage(std::true_type{}, st + 1, sK1, sV1, sK0, sV0);
+    } else {
+      stage(std::true_type{}, st, sK0, sV0, sK1, sV1);
+    }
   }
-  if (st < ns) stage(st, sK0, sV0, sK1, sV1);
 
   // lane holds O[row][16d + 4lg + (0..3)]; lane groups lg and lg^1 trade
   // halves so that each lane stores 8 consecutive channels; rows >= N drop
