@@ -7,7 +7,7 @@ import torch
 from oracle import torch_ref
 from tests.cases import ROPE_BASE, TOL_MEAN
 from tests.test_gpu_parity import _compare
-from triton_fused_rope_flash_attn_amd import CosSinTable, _lib, sdpa_triton_fa_rope
+from triton_fused_rope_flash_attn_amd import CosSinTable, RoPEAttention, _lib, sdpa_triton_fa_rope
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -84,3 +84,53 @@ def test_wide_planes_of_small_calls(side, has_cls, dt, B):
     got = (o.detach(), *torch.autograd.grad(o, leaves, do))
     ref = torch_ref.forward_backward(*(t.detach().float() for t in (q, k, v)), do.float(), *table.tables(), has_cls)
     _compare(f"wide-N{N}-B{B}", got, ref, out_dtype=dt)
+
+
+def _overlapping_rows(B, H, N, D, dt, gen, stride):
+    """dO with one row stride for all rows: 0 (one row for every token, as the
+    backward of a sum over the tokens gives it) or less than D (rows overlap)."""
+    base = torch.randn(B, H, (N - 1) * stride + D, generator=gen).to(dt).to(DEV)
+    return base.as_strided((B, H, N, D), (*base.stride()[:2], stride, 1))
+
+
+# rows past the plane's end in the last 32-row block: 27 (N = 37), none (64), 31
+# (65), 27 (197); few planes, so that the short kernels take them
+@pytest.mark.parametrize("side,has_cls", [(6, True), (8, False), (8, True), (14, True)])
+@pytest.mark.parametrize("D,io", [(64, "bf16"), (32, "fp16"), (32, "amp"), (64, "fp32"), (64, "amp"), (32, "fp32")])
+@pytest.mark.parametrize("stride", [0, 16])
+def test_short_planes_overlapping_dout_rows(side, has_cls, D, io, stride):
+    B, H, N = 2, 3, side * side + int(has_cls)
+    dt = DT[io]
+    print(f"short planes, dO row stride {stride}, N={N} D={D} {io}", flush=True)
+    g = torch.Generator().manual_seed(63)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    q, k, v = (torch.randn(B, H, N, D, generator=g).to(dt).to(DEV).requires_grad_() for _ in range(3))
+    do = _overlapping_rows(B, H, N, D, dt, g, stride)
+    with torch.autocast("cuda", torch.bfloat16, enabled=io == "amp"):
+        o = sdpa_triton_fa_rope(q, k, v, table, H_img=side, has_cls=has_cls)
+    got = (o.detach(), *torch.autograd.grad(o, (q, k, v), do))
+    ref = torch_ref.forward_backward(*(t.detach().float() for t in (q, k, v)), do.float().contiguous(), *table.tables(),
+                                     has_cls)
+    tag = f"short-{io}-N{N}-D{D}-dOstride{stride}"
+    if io == "fp32":
+        # the split products' error grows with the entries: the bound for entries of unit size, times the largest
+        big = max(1.0, ref[3].abs().max().item())
+        _compare(tag, got, ref, tol_max=1e-4 * big, tol_mean=1e-5 * big)
+    else:
+        # (the gradients' bounds grow with their size: twice the error of storing them in the compute type)
+        _compare(tag, got, ref, tol_mean=2e-3 if io == "amp" else TOL_MEAN, out_dtype=torch.bfloat16 if io == "amp" else dt)
+
+
+def test_token_sum_pooling():
+    """The backward of a sum over the tokens, whose gradient has a row stride of 0,
+    through the layer's packed op, against the same gradient in memory of its own."""
+    torch.manual_seed(64)
+    layer = RoPEAttention(192, 3, H_img=6, device=DEV, dtype=torch.bfloat16)
+    layer.proj = torch.nn.Identity()
+    x = torch.randn(2, 37, 192, device=DEV).bfloat16().requires_grad_()
+    w = torch.randn(2, 192, device=DEV).bfloat16()
+    out = layer(x)
+    leaves = (x, layer.qkv.weight)
+    got = torch.autograd.grad(out.sum(1), leaves, w, retain_graph=True)
+    want = torch.autograd.grad(out, leaves, w[:, None, :].repeat(1, 37, 1))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))

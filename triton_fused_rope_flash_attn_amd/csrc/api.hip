@@ -87,7 +87,6 @@ int check_ptr(const void* p, int es) {
   return FAROPE_OK;
 }
 
-// 16-byte vector path allowed: unit channel stride and 16-byte aligned rows.
 // 16-byte vector access: unit d-stride, 16-byte aligned base and strides, a
 // non-negative row stride, and every byte offset inside one (b, h) plane
 // (row n, channel d) below 2^31, so kernels can address a plane as 64-bit
@@ -95,7 +94,10 @@ int check_ptr(const void* p, int es) {
 // the plane that the kernels address unconditionally (their blocks of up to
 // 256 rows end past N): those offsets must stay below 2^31 too, so that they
 // fall outside the descriptor range (loads read 0, stores are dropped)
-// instead of wrapping around to a row of the plane.
+// instead of wrapping around to a row of the plane.  Rows of an input may
+// overlap (0 <= s[2] < head_dim, e.g. dO of a sum over the tokens): rows past
+// the plane can then lie inside the range, so a kernel must not count on the
+// zeros of an input alone.
 constexpr int kRowPad = 256;
 int vec_ok(const void* p, const int64_t s[4], int es, int n_rows, int head_dim) {
   if (s[3] != 1) return 0;

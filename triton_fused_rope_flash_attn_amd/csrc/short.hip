@@ -416,8 +416,13 @@ __global__ void __launch_bounds__(64 * kShortNW) bwd_short_kernel(const BwdParam
   }
 
   own_rows<IO, CT, D>(K, V, T, p.scale_log2, row, lg, fa, fb, rb);
-  // -LSE2 of the staged rows (rows >= N read 0: their Q-hat and dO rows are zero and add nothing)
-  if (tid < 32 * NB) sNl[tid] = -kLog2e * __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rL, (unsigned)tid * 4u, 0u, 0));
+  // -LSE2 of the staged rows; -inf for rows >= N, whose P is then 0.  (Their dO
+  // rows read 0 only where dO's rows do not overlap: with a row stride of 0, as
+  // the backward of a sum over the tokens gives it, they read the one real row.)
+  if (tid < 32 * NB) {
+    const float ls = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rL, (unsigned)tid * 4u, 0u, 0));
+    sNl[tid] = tid < N ? -kLog2e * ls : -INFINITY;
+  }
   stage_plane<IO, CT, D, NB>(Q, G, &O, T, 1.f, N, tid, sA, sB, sNd);
   lds_barrier();
   if (row - lr >= N) return;   // wave-uniform; no barrier follows
