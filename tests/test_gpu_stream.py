@@ -114,3 +114,27 @@ def test_streamed_tiles_large_logits():
     for name, x, y in zip(("O", "LSE", "dQ", "dK", "dV"), got, plain):
         assert torch.isfinite(x).all(), name
         assert _rel(x, y) < (1e-6 if name == "LSE" else BF16_PATHS), f"{name}: {_rel(x, y):.2e}"
+
+
+# dO with one row stride for all rows: 0 (one row for every token, as the backward
+# of a sum over the tokens gives it) or less than D (rows overlap); both tile sizes;
+# N = 289, 324, 400, 577, 1025: 31, 28, 16, 31, 31 rows past the plane's end in the
+# last 32-row block, and 290 and 257 in D 32
+@pytest.mark.parametrize("stride", [0, 16])
+@pytest.mark.parametrize("side,has_cls,D,dt,B", [
+    (17, False, 64, "bf16", 2), (18, False, 64, "fp16", 2), (24, True, 64, "bf16", 2), (32, True, 64, "bf16", 1),
+    (24, True, 64, "bf16", 44), (16, True, 32, "bf16", 2), (17, True, 32, "fp16", 2), (16, True, 32, "bf16", 100),
+    (17, False, 128, "fp16", 2), (20, False, 128, "fp16", 2), (24, True, 128, "fp16", 2),
+])
+def test_streamed_tiles_overlapping_dout_rows(side, has_cls, D, dt, B, stride):
+    H, N = 3, side * side + int(has_cls)
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
+    print(f"streamed, dO row stride {stride}, N={N} D={D} B={B} {dt}", flush=True)
+    g = torch.Generator().manual_seed(44)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    q, k, v, _ = _views(B, H, N, D, dt, g)
+    base = torch.randn(B, H, (N - 1) * stride + D, generator=g).to(dt).to(DEV)
+    do = base.as_strided((B, H, N, D), (*base.stride()[:2], stride, 1))
+    got = _run(q, k, v, do, table, has_cls)
+    ref = torch_ref.forward_backward(*(t.float().contiguous() for t in (q, k, v, do)), *table.tables(), has_cls)
+    _compare(f"streamed-N{N}-D{D}-dOstride{stride}", (got[0], *got[2:]), ref, out_dtype=dt)

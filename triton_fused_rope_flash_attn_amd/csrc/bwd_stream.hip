@@ -243,9 +243,12 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) s
 }
 
 // ---------------------------------------------------------------------------
-// dK / dV of 128-key tiles (64 with KT = 1).  Wave w owns KT 16-key subtiles: K-hat and V rows are B operands in registers, dK-hat and dV
-// accumulate in registers.  Queries >= N have zero Q-hat and dO rows and
-// -LSE2 = -delta = 0 (reads past the range), so they add nothing.
+// dK / dV of 128-key tiles (64 with KT = 1).  Wave w owns KT 16-key subtiles:
+// K-hat and V rows are B operands in registers, dK-hat and dV accumulate in
+// registers.  In the last stage queries >= N take -LSE2 = -inf, so that P = 0.
+// (Their Q-hat, -LSE2 and -delta read 0 past the range; their dO does so only
+// where dO's rows do not overlap: with a row stride of 0, as the backward of a
+// sum over the tokens gives it, every row reads the one real row.)
 // ---------------------------------------------------------------------------
 template <typename S, int CT, int D, int KT>
 __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const BwdParams p) {
@@ -310,11 +313,16 @@ __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const Bw
   for (int d = 0; d < DT; ++d) to[d] = swz<D>(4 * lg + (lr >> 2), 16 * d + 4 * (lr & 3));
 
   using Acc = f32x4[KT][2];
-  auto sp = [&](const S* __restrict__ q, const S* __restrict__ g, const float* __restrict__ l, const float* __restrict__ dl,
-                Acc& sacc, Acc& pacc) __attribute__((always_inline)) {
+  // last: queries at left or beyond (counted from the block's first) do not exist
+  auto sp = [&](auto last, int left, const S* __restrict__ q, const S* __restrict__ g, const float* __restrict__ l,
+                const float* __restrict__ dl, Acc& sacc, Acc& pacc) __attribute__((always_inline)) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const f32x4 nl = *reinterpret_cast<const f32x4*>(l + 16 * h + 4 * lg);
+      f32x4 nl = *reinterpret_cast<const f32x4*>(l + 16 * h + 4 * lg);
+      if constexpr (last.value) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) nl[i] = 16 * h + 4 * lg + i < left ? nl[i] : -INFINITY;
+      }
       const f32x4 nd = *reinterpret_cast<const f32x4*>(dl + 16 * h + 4 * lg);
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
@@ -358,15 +366,16 @@ __global__ void __launch_bounds__(kStreamNW * 64, 2) stream_dkdv_kernel(const Bw
     stage_barrier();
     if (!last.value) load(st + 1, qn, gn, ln, dn);
     if (active) {
+      const int left = N - st * SR;
       Acc sA, pA;
-      if (!last.value || st * SR + 32 < N) {
+      if (!last.value || left > 32) {
         Acc sB, pB;
-        sp(q, g, l, dl, sA, pA);
-        sp(q + 32 * D, g + 32 * D, l + 32, dl + 32, sB, pB);
+        sp(last, left, q, g, l, dl, sA, pA);
+        sp(last, left - 32, q + 32 * D, g + 32 * D, l + 32, dl + 32, sB, pB);
         out(q, g, sA, pA);
         out(q + 32 * D, g + 32 * D, sB, pB);
       } else {
-        sp(q, g, l, dl, sA, pA);
+        sp(last, left, q, g, l, dl, sA, pA);
         out(q, g, sA, pA);
       }
     }
