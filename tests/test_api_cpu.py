@@ -230,3 +230,37 @@ def test_residual_rule_matches_library():
                 n = _lib.residual_elems(desc)
                 assert (n > 0) == attention._uses_residual(io, ct, D), (io, ct, D)
                 assert n in (0, 2 * 3 * 197 * D)
+
+
+@pytest.mark.parametrize("qkv,error,match", [
+    # [B * N, 3 C] holds the same values: taken, up to the device check
+    (lambda m: lambda x: m(x).flatten(0, 1), RuntimeError, "ROCm GPUs only"),
+    # twice as wide: not q, k and v of num_heads heads of head_dim, whatever head_dim the width allows
+    (lambda m: lambda x: m(x).repeat(1, 1, 2), RuntimeError, "invalid for input of size"),
+    (lambda m: lambda x: m(x)[:, :-1], RuntimeError, "invalid for input of size"),
+], ids=["flat", "wide", "short"])
+def test_block_takes_and_refuses_qkv_outputs_of_other_shapes(qkv, error, match):
+    """A replaced qkv projection: its output counts by its elements, as for the
+    [B, N, 3, H, D] view of it."""
+    from triton_fused_rope_flash_attn_amd import RoPEAttention
+
+    blk = RoPEAttention(128, 2, H_img=4, has_cls=True, device="cpu")
+    blk.rope = CosSinTable(100.0, 4, 128, device="cpu") if match.startswith("invalid") else blk.rope
+    proj = blk.qkv
+
+    class Replaced(torch.nn.Module):
+        def forward(self, x):
+            return qkv(proj)(x)
+
+    blk.qkv = Replaced()
+    with pytest.raises(error, match=match):
+        blk(torch.randn(2, 17, 128))
+
+
+def test_block_refuses_a_head_dim_that_is_not_the_projections():
+    from triton_fused_rope_flash_attn_amd import RoPEAttention
+
+    blk = RoPEAttention(128, 2, H_img=4, has_cls=True, device="cpu")
+    blk.head_dim = 32
+    with pytest.raises(RuntimeError, match="invalid for input of size"):
+        blk(torch.randn(2, 17, 128))

@@ -52,9 +52,10 @@ class RoPEAttention(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         B, N, C = x.shape
         qkv = self.qkv(x)
-        if self.attn is sdpa_triton_fa_rope:
+        if self.attn is sdpa_triton_fa_rope and qkv.shape == (B, N, 3 * self.num_heads * self.head_dim):
             # the kernels read and write the projections' own layouts: the views
-            # below cost a copy of O and two of the gradients (64 x 197 x 384: 66 us)
+            # below cost a copy of O and two of the gradients (64 x 197 x 384: 66 us);
+            # an output of another shape is left to the view, which takes or refuses it
             return self.proj(packed_attention(qkv, self.rope, self.num_heads, self.H_img, self.has_cls))
         qkv = qkv.view(B, N, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4)
         q, k, v = qkv.unbind(0)   # [B, H, N, D] views with strides (N*3C, D, 3C, 1)
