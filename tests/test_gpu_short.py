@@ -134,3 +134,23 @@ def test_token_sum_pooling():
     got = torch.autograd.grad(out.sum(1), leaves, w, retain_graph=True)
     want = torch.autograd.grad(out, leaves, w[:, None, :].repeat(1, 37, 1))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("D,io", [(64, "bf16"), (32, "bf16"), (32, "fp16"), (32, "amp"), (64, "fp32"), (32, "fp32")])
+@pytest.mark.parametrize("what", ["q", "k"])
+@pytest.mark.parametrize("side", [6, 14])
+def test_short_planes_nan_reaches_every_gradient(side, what, D, io):
+    """A NaN in one query (or key) makes that query's (every query's) probabilities
+    NaN, and with them every key's dV; the other plane stays finite."""
+    N = side * side
+    g = torch.Generator(device=DEV).manual_seed(65)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    t = dict(zip("qkv", (torch.randn(1, 2, N, D, generator=g, device=DEV).to(DT[io]) for _ in range(3))))
+    t[what][0, 0, 5, 3] = float("nan")
+    leaves = [t[c].requires_grad_() for c in "qkv"]
+    with torch.autocast("cuda", torch.bfloat16, enabled=io == "amp"):
+        o = sdpa_triton_fa_rope(*leaves, table, H_img=side, has_cls=False)
+    dq, dk, dv = torch.autograd.grad(o, leaves, torch.randn(1, 2, N, D, generator=g, device=DEV).to(DT[io]))
+    assert dv[0, 0].isnan().all() and dk[0, 0].isnan().all()
+    assert dq[0, 0, 5].isnan().all() if what == "q" else dq[0, 0].isnan().all()
+    assert all(torch.isfinite(x[0, 1]).all() for x in (o, dq, dk, dv))

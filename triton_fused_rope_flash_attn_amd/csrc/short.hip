@@ -416,6 +416,8 @@ __global__ void __launch_bounds__(64 * kShortNW) bwd_short_kernel(const BwdParam
   }
 
   own_rows<IO, CT, D>(K, V, T, p.scale_log2, row, lg, fa, fb, rb);
+  // P needs no clamp here (which would turn a NaN into 0): keys >= N of a lane
+  // only reach rows that are never stored.
   // -LSE2 of the staged rows; -inf for rows >= N, whose P is then 0.  (Their dO
   // rows read 0 only where dO's rows do not overlap: with a row stride of 0, as
   // the backward of a sum over the tokens gives it, they read the one real row.)
@@ -445,7 +447,7 @@ __global__ void __launch_bounds__(64 * kShortNW) bwd_short_kernel(const BwdParam
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        pv[4 * h + i] = __builtin_amdgcn_fmed3f(fast_exp2(sacc[i]), 0.f, 1.f);
+        pv[4 * h + i] = fast_exp2(sacc[i]);
         dsv[4 * h + i] = pv[4 * h + i] * pacc[i];
       }
     }
