@@ -251,20 +251,26 @@ int farope_attn_bwd_noalloc(const farope_attn_desc* desc,
 
 /*
  * Tile table query (replaces the reference's triton.autotune configs,
- * FA:76-90, FA:318-324, FA:359-373, FA:693-707).  which: 0 = forward,
- * 1 = backward.  out[0] = variant (fwd: 0 = persistent pipelined kernel,
- * 1 = one wave per (b, h) plane for 193 <= N <= 208 at head_dim 64 with
- * 16-bit tensors, assuming vector access (the streamed query tiles of
- * farope_attn_fwd_ws and, in either pass, the 64-row short-plane kernels that
- * take calls of few or short planes at head_dim 32 and 64 are not reported, nor
- * the 128-row items of forward calls of few planes at head_dim 128); bwd: 0 fused, 1 split, 2 split with
- * the key-tile kernel, 3 key tiles that store dS and dQ as one GEMM over it,
- * 4 streamed tiles, assuming vector access), out[1] = query (fwd) or key (bwd) rows per work item,
- * out[2] = work items per (b, h) plane, out[3] = threads per workgroup.  When 1 to 8 rows are left past out[1] * out[2] (N = 1025 with
- * 128- or 256-row items), they are computed by the tail-row kernels (or, for
- * a single row with fp16 logit operands, by one designated item of each plane
- * in the forward and dQ block kernels) rather than by one more, nearly
- * empty, work item.
+ * FA:76-90, FA:318-324, FA:359-373, FA:693-707).
+ *
+ * which = 0, 1: the general kernels of a forward (0) or backward (1) call.
+ * which = 2, 3: the kernels that such a call takes, vector access to every
+ * tensor and, in the forward, a workspace (farope_attn_fwd_ws) assumed.
+ *
+ * out[0] = variant.  Forward: 0 persistent pipelined tiles, 1 one wave per
+ * (b, h) plane (193 <= N <= 208 at head_dim 64, 16-bit tensors); with which = 2
+ * also 2 streamed tiles, 3 short-plane kernels.  Backward: 0 one pass, 1 split,
+ * 2 split with the key-tile kernel, 3 key tiles that store dS and dQ as one GEMM
+ * over it, 4 streamed tiles; with which = 3 also 5 short-plane kernels.
+ * out[1] = query (forward) or key (backward) rows per work item (which = 0: not
+ * counting that calls of few planes at head_dim 128 take 128-row items),
+ * out[2] = work items per (b, h) plane, out[3] = threads per workgroup.
+ *
+ * When 1 to 8 rows are left past out[1] * out[2] (N = 1025 with 128- or
+ * 256-row items), they are computed by the tail-row kernels (or, for a single
+ * row with fp16 logit operands, by one designated item of each plane in the
+ * forward and dQ block kernels) rather than by one more, nearly empty, work
+ * item.
  */
 int farope_tile_config(const farope_attn_desc* desc, int32_t which, int32_t out[4]);
 

@@ -154,3 +154,18 @@ def test_short_planes_nan_reaches_every_gradient(side, what, D, io):
     assert dv[0, 0].isnan().all() and dk[0, 0].isnan().all()
     assert dq[0, 0, 5].isnan().all() if what == "q" else dq[0, 0].isnan().all()
     assert all(torch.isfinite(x[0, 1]).all() for x in (o, dq, dk, dv))
+
+
+def test_more_planes_than_a_launch_of_tiles_holds():
+    """2^24 planes of one row (1 GB a tensor): the softmax over one key is 1, so O = V."""
+    B, D = 2 ** 24, 32
+    print(f"{B} planes of one row", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(66)
+    q, k, v = (torch.randn(B, 1, 1, D, generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(3))
+    table = CosSinTable(ROPE_BASE, 1, D, device=DEV)
+    o, lse, _ = torch.ops.farope.attn_fwd(q, k, v, table.packed(), 1, False, D ** -0.5, _lib.BF16)
+    assert torch.equal(o, v)
+    # K-hat * c2 is rounded to bf16, by at most 2^-9 of each term of the logit (twice that
+    # leaves room for the fp32 arithmetic)
+    terms = q.float() * k.float() * D ** -0.5
+    assert ((lse - terms.sum(-1)).abs() <= 2.0 ** -8 * terms.abs().sum(-1) + 1e-6).all()

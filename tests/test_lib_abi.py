@@ -83,6 +83,45 @@ def test_tile_table(lib, N, D, has_cls, fwd_var, fwd_items, bwd_var):
     assert f[3] % 64 == 0 and b[3] % 64 == 0
 
 
+def _route(planes, N, D, io, ct, which):
+    """Variant and rows per item of a forward (which = 2) or backward (3) call with vector access."""
+    has_cls = N > 1 and int((N - 1) ** 0.5) ** 2 == N - 1
+    desc = _lib.make_desc(planes, 1, N, D, N - int(has_cls), has_cls, io, ct, D ** -0.5)
+    return _lib.tile_config(desc, which)[:2]
+
+
+@pytest.mark.parametrize("planes,N,D,io,ct,fwd,bwd", [
+    (12, 197, 64, _lib.BF16, _lib.BF16, (3, 64), (5, 64)),
+    (3072, 197, 64, _lib.BF16, _lib.BF16, (1, 208), (0, 256)),
+    (1536, 256, 64, _lib.BF16, _lib.BF16, (0, 256), (0, 256)),
+    (12, 257, 64, _lib.BF16, _lib.BF16, (2, 64), (1, 256)),
+    (384, 577, 64, _lib.BF16, _lib.BF16, (2, 128), (4, 128)),
+    (16, 197, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (24, 1025, 128, _lib.BF16, _lib.BF16, (0, 128), (3, 128)),
+    (384, 1025, 128, _lib.BF16, _lib.BF16, (0, 256), (3, 128)),
+])
+def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
+    """which = 2 and 3: the kernels that a call takes."""
+    assert _route(planes, N, D, io, ct, 2) == fwd
+    assert _route(planes, N, D, io, ct, 3) == bwd
+
+
+def test_routes_stay_within_the_launch_limit(lib):
+    """A launch holds fewer than 2^32 threads: calls whose tiles need 2^24 workgroups
+    of 256 keep the kernels that take any number of planes (the largest tensors
+    here are 4 GB)."""
+    m = 2 ** 24
+    for io in (_lib.BF16, _lib.F32):
+        assert _route(m - 1, 4, 32, io, io, 2)[0] == 3 and _route(m, 4, 32, io, io, 2)[0] == 0
+        assert _route(m // 2 - 1, 4, 32, io, io, 3)[0] == 5 and _route(m // 2, 4, 32, io, io, 3)[0] == 1
+    # head_dim 128: the K-hat pass takes 17 blocks of 16 rows per two planes of 257 rows
+    n = 2 * (m - 1) // 17
+    for planes, streamed in ((n - 1, True), (n + 3, False)):
+        assert (_route(planes, 257, 128, _lib.F16, _lib.F16, 2)[0] == 2) == streamed
+        desc = _lib.make_desc(planes, 1, 257, 128, 256, True, _lib.F16, _lib.F16, 0.1)
+        assert (_lib.fwd_workspace_elems(desc) != 0) == streamed
+
+
 def _ds_elems(B, H, N, D):
     """Workspace of the stored-dS backward (None where it does not apply: more
     than one key past the 128-key tiles, or a dS^T plane larger than 16 Q

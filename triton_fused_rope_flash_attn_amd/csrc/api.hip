@@ -323,7 +323,9 @@ bool stream_shape(const farope_attn_desc* d) {
   if (d->io_dtype == FAROPE_F32 || d->io_dtype != d->compute_dtype) return false;
   // (head_dim 128 with bf16 compute takes fp16 logit operands: other kernels)
   if (d->head_dim != 64 && d->head_dim != 32 && !(d->head_dim == 128 && d->compute_dtype == FAROPE_F16)) return false;
-  return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kStreamTileRows / 2) <= INT32_MAX;
+  const int64_t planes = (int64_t)d->batch * d->heads;
+  return planes * cdiv(d->seq_len, kStreamTileRows / 2) <= kMaxWorkgroups &&
+         khat_blocks(planes, d->seq_len, d->head_dim) <= kMaxWorkgroups;
 }
 // Forward: planes past the 256 rows whose table fwd_kernel keeps in LDS.
 // Measured (us, fwd_kernel / streamed, the K-hat pass included): D 64, N 577,
@@ -342,16 +344,33 @@ bool fwd_stream(const farope_attn_desc* d) { return stream_shape(d) && d->seq_le
 bool bwd_stream(const farope_attn_desc* d) {
   return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim >= 64 ? 1 : 0);
 }
-// The short-plane kernels (short.hip): tensors in the compute type or in fp32,
-// head_dim 32 or 64, N <= 256.  (Vector access to every tensor is checked at
-// the call.)  short_tiles: their 64-row tiles over the whole call.
-bool short_shape(const farope_attn_desc* d) {
-  if (d->io_dtype != FAROPE_F32 && d->io_dtype != d->compute_dtype) return false;
-  if (d->head_dim != 64 && d->head_dim != 32) return false;
-  return d->seq_len <= kPlaneMaxN && (int64_t)d->batch * d->heads * 2 * cdiv(d->seq_len, kShortTileRows) <= INT32_MAX;
+// Its workspace, in fp32 elements, each part from a 256-byte boundary:
+// -delta rows, -LSE2 rows, Q-hat rows and K-hat * c2 rows (16-bit).
+struct StreamWs {
+  int64_t nl, qhat, khat, total;
+};
+StreamWs stream_ws(const farope_attn_desc* d) {
+  const int64_t rows = (int64_t)d->batch * d->heads * d->seq_len;
+  auto al = [](int64_t x) { return (x + 63) & ~int64_t(63); };
+  StreamWs w{};
+  w.nl = al(rows);
+  w.qhat = al(w.nl + rows);
+  w.khat = al(w.qhat + rows * d->head_dim / 2);
+  w.total = w.khat + rows * d->head_dim / 2;
+  return w;
 }
+
+// The short-plane kernels (short.hip): tensors in the compute type or in fp32,
+// head_dim 32 or 64, N <= 256, and a launch of `per` workgroups per tile.
+// (Vector access to every tensor is checked at the call.)  short_tiles: their
+// 64-row tiles over the whole call.
 int64_t short_tiles(const farope_attn_desc* d) {
   return (int64_t)d->batch * d->heads * cdiv(d->seq_len, kShortTileRows);
+}
+bool short_shape(const farope_attn_desc* d, int per) {
+  if (d->io_dtype != FAROPE_F32 && d->io_dtype != d->compute_dtype) return false;
+  if (d->head_dim != 64 && d->head_dim != 32) return false;
+  return d->seq_len <= kPlaneMaxN && short_tiles(d) * per <= kMaxWorkgroups;
 }
 // Forward: up to 128 rows always, longer planes while the call has too few of
 // them to fill the chip with one workgroup (fwd_kernel) or one wave
@@ -364,7 +383,7 @@ int64_t short_tiles(const farope_attn_desc* d) {
 // 512 x 197 14.3 / 14.0, 4096 x 197 84 / 87; fp32 compute 512 x 197 29.9 / 30.1,
 // 4096 x 144 162 / 168.
 bool fwd_short(const farope_attn_desc* d) {
-  if (!short_shape(d)) return false;
+  if (!short_shape(d, 1)) return false;
   if (d->seq_len <= 128) return true;
   const int64_t t = short_tiles(d);
   const bool f32 = d->compute_dtype == FAROPE_F32;
@@ -384,27 +403,12 @@ bool fwd_short(const farope_attn_desc* d) {
 // 4096 x 64 97 / 67, 1024 x 197 82 / 97; D 64 48 x 197 26.0 / 17.9, 3072 x 64
 // 91 / 113.
 bool bwd_short(const farope_attn_desc* d) {
-  if (!short_shape(d)) return false;
+  if (!short_shape(d, 2)) return false;
   if (d->compute_dtype == FAROPE_F32) return true;
   const bool io16 = d->io_dtype != FAROPE_F32, one = d->seq_len <= kShortTileRows;
   if (d->head_dim == 64 && d->seq_len <= 32) return false;
   if (d->head_dim == 32 ? io16 || one : io16 && one) return true;
   return 2 * short_tiles(d) <= 512;
-}
-// Its workspace, in fp32 elements, each part from a 256-byte boundary:
-// -delta rows, -LSE2 rows, Q-hat rows and K-hat * c2 rows (16-bit).
-struct StreamWs {
-  int64_t nl, qhat, khat, total;
-};
-StreamWs stream_ws(const farope_attn_desc* d) {
-  const int64_t rows = (int64_t)d->batch * d->heads * d->seq_len;
-  auto al = [](int64_t x) { return (x + 63) & ~int64_t(63); };
-  StreamWs w{};
-  w.nl = al(rows);
-  w.qhat = al(w.nl + rows);
-  w.khat = al(w.qhat + rows * d->head_dim / 2);
-  w.total = w.khat + rows * d->head_dim / 2;
-  return w;
 }
 
 // Caller workspace of farope_attn_bwd: enough for whichever path the call
@@ -633,16 +637,32 @@ int farope_tile_config(const farope_attn_desc* desc, int32_t which, int32_t out[
   FAROPE_TRY(check_desc(desc));
   if (!out) return FAROPE_ERR_NULL;
   const int D = desc->head_dim, N = desc->seq_len;
-  if (which == 0) {
+  if (which == 2 && fwd_short(desc)) {
+    out[0] = FWD_SHORT;
+    out[1] = kShortTileRows;
+    out[2] = cdiv(N, kShortTileRows);
+    out[3] = kShortThreads;
+  } else if (which == 2 && !fwd_plane(desc, true) && fwd_stream(desc)) {
+    out[0] = FWD_STREAM;
+    out[1] = stream_rows(desc->batch * desc->heads, N, D, false);
+    out[2] = cdiv(N, out[1]);
+    out[3] = kStreamThreads;
+  } else if (which == 3 && bwd_short(desc)) {
+    out[0] = BWD_SHORT;
+    out[1] = kShortTileRows;
+    out[2] = cdiv(N, kShortTileRows);
+    out[3] = kShortThreads;
+  } else if (which == 0 || which == 2) {
     if (fwd_plane(desc, true)) {
-      out[0] = 1;
+      out[0] = FWD_PLANE;
       out[1] = fwd_plane_rows();
       out[2] = 1;
       out[3] = fwd_plane_threads();
       return FAROPE_OK;
     }
-    const int rows = fwd_block_rows(D, desc->io_dtype, desc->compute_dtype);
-    out[0] = 0;
+    const int rows = which == 2 ? fwd_call_rows(D, desc->io_dtype, desc->compute_dtype, desc->batch * desc->heads, N)
+                                : fwd_block_rows(D, desc->io_dtype, desc->compute_dtype);
+    out[0] = FWD_TILES;
     out[1] = rows;
     out[2] = main_blocks(desc->batch * desc->heads, N, rows);
     out[3] = fwd_threads(D);

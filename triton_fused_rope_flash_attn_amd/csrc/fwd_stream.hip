@@ -34,8 +34,6 @@ namespace farope {
 // 38.2 -> 37.1; 512 of N 257, D 32 24.3 -> 22.6; 384 of N 577, D 128 120.4 ->
 // 117.7.  One plane: 37.0, 22.8, 120.1; four: 37.9, 22.8, 118.0.
 // ---------------------------------------------------------------------------
-constexpr int kKhatPlanes = 2;
-
 template <typename S, int CT, int D>
 __global__ void __launch_bounds__(256) stream_khat_kernel(const KhatParams p, int n_blk) {
   constexpr int CPR = D / 8, ROWS = 256 / CPR;
@@ -308,7 +306,7 @@ __global__ void __launch_bounds__(kStreamNW * 64, D == 128 && QT == 2 ? 2 : 3) f
 template <typename S, int CT>
 static hipError_t khat_launch(const KhatParams& p, int D, hipStream_t st) {
   const int rows = 256 / (D / 8), n_blk = (p.N + rows - 1) / rows;
-  const int n_wg = n_blk * ((p.planes + kKhatPlanes - 1) / kKhatPlanes);
+  const int n_wg = (int)khat_blocks(p.planes, p.N, D);
   auto kern = D == 128 ? stream_khat_kernel<S, CT, 128> : D == 64 ? stream_khat_kernel<S, CT, 64> : stream_khat_kernel<S, CT, 32>;
   hipLaunchKernelGGL(kern, dim3(n_wg), dim3(256), 0, st, p, n_blk);
   return hipGetLastError();

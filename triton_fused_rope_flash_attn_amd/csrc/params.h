@@ -75,7 +75,18 @@ enum BwdVariant : int {
                     // (bwd_ds.hip; with vector access to every tensor, else BWD_SPLIT16)
   BWD_STREAM = 4,   // streamed dQ tiles, then streamed dK/dV tiles (bwd_stream.hip;
                     // with vector access to every tensor, else BWD_SPLIT)
+  BWD_SHORT = 5,    // short-plane kernels, dQ and dK/dV in one launch (short.hip;
+                    // with vector access to every tensor, else as without them)
 };
+enum FwdVariant : int {
+  FWD_TILES = 0,    // persistent query tiles (fwd.hip)
+  FWD_PLANE = 1,    // one wave per plane (fwd_plane.hip)
+  FWD_STREAM = 2,   // streamed query tiles (fwd_stream.hip)
+  FWD_SHORT = 3,    // short-plane kernel (short.hip)
+};
+
+// Workgroups of 256 threads a launch may hold: HIP refuses 2^32 threads or more.
+constexpr int64_t kMaxWorkgroups = (int64_t(1) << 24) - 1;
 
 // Launchers: return hipSuccess or the launch error.  io/ct are DT_* codes.
 hipError_t launch_fwd(const FwdParams& p, int io, int ct, int D, hipStream_t st);
@@ -154,14 +165,21 @@ struct KhatParams {
   int planes, H, N, has_cls;
   float c2;            // softmax_scale * log2(e)
 };
+constexpr int kKhatPlanes = 2;   // planes per workgroup (see stream_khat_kernel)
+inline int64_t khat_blocks(int64_t planes, int N, int D) {
+  const int rows = 256 / (D / 8);
+  return (int64_t)((N + rows - 1) / rows) * ((planes + kKhatPlanes - 1) / kKhatPlanes);
+}
 hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st);
 // Forward over 128-query tiles; khat from launch_stream_khat.
 hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st);
 hipError_t launch_bwd_stream(const BwdParams& p, int io, int D, hipStream_t st);
 
-// Short planes (short.hip): head_dim 32 or 64, N <= 256, 16-bit compute, vector
-// access to every tensor; 64 rows per workgroup, the backward in one launch.
+// Short planes (short.hip): head_dim 32 or 64, N <= 256, tensors in the compute
+// type or in fp32, vector access to every tensor; 64 rows per workgroup, the
+// backward in one launch.
 constexpr int kShortTileRows = 64;
+constexpr int kShortThreads = 256;
 hipError_t launch_fwd_short(const FwdParams& p, int io, int ct, int D, hipStream_t st);
 hipError_t launch_bwd_short(const BwdParams& p, int io, int ct, int D, hipStream_t st);
 

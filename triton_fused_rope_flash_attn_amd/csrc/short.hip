@@ -32,6 +32,7 @@ namespace farope {
 namespace {
 constexpr int kShortNW = 4;
 constexpr int kShortRows = 16 * kShortNW;   // rows of a workgroup
+static_assert(kShortRows == kShortTileRows && 64 * kShortNW == kShortThreads, "");
 }  // namespace
 
 // Staged operands: 16-bit compute keeps one tile of its type; fp32 compute
