@@ -362,6 +362,26 @@ def test_split_backward_io_variants(side, has_cls, D, mode):
         _compare(tag, ours, ref, out_dtype=dtype)
 
 
+@pytest.mark.parametrize("D,B,H", [(32, 25, 8), (64, 25, 8)])
+@pytest.mark.parametrize("side,has_cls", [(17, False), (20, False), (20, True)])
+def test_fp32_split_backward_of_many_tiles(side, has_cls, D, B, H):
+    """The dK/dV kernel in fp32 compute past 2 tiles per CU reads its fragments per
+    key subtile: the same values as a call of few planes, bit for bit.
+    N = 289, 400, 401: 33, 16, 17 keys of the last 128-key tile."""
+    N = side * side + int(has_cls)
+    assert B * H * -(-N // 128) > 512
+    cfg = dict(B=B, H=H, side=side, has_cls=has_cls, D=D, dtype=torch.float32, scale=1.0, dout="randn")
+    _say(f"case many fp32 tiles: {cfg}")
+    q, k, v, do = make_inputs(cfg, DEV, seed=8)
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    many = _run_ours(q, k, v, do, table, has_cls)
+    few = _run_ours(*(t[-2:] for t in (q, k, v, do)), table, has_cls)
+    for name, a, b in zip(("O", "dQ", "dK", "dV"), many, few):
+        assert torch.isfinite(a).all() and torch.equal(a[-2:], b), name
+    ref = _ref(*(t[:2] for t in (q, k, v, do)), table, has_cls)
+    _compare(f"many-fp32-tiles-N{N}-D{D}", [t[:2] for t in many], ref, tol_max=1e-4, tol_mean=1e-5)
+
+
 def test_stride0_dout_from_sum():
     cfg = dict(CONFIGS["vit_b"], B=4)
     q, k, v, _ = make_inputs(cfg, DEV)

@@ -752,7 +752,12 @@ bwd_dq_kernel(const BwdParams p) {
 // bf16 Q-hat of the dK product is that value divided by c2.  A pass whose
 // fp16 rows overflowed (inf) or underflowed (max below 2^-10) rotates Q
 // again (raw), and a rescaled pass does too.
-template <typename IO, int CT, int D, int NW, int KT, int QS, bool VEC, bool FS, bool HAT>
+// KU: key subtiles that share one read of each Q-hat / dO fragment (KT, or 1).
+// Shared reads relieve the LDS, but hold KU subtiles' products at once: in fp32
+// compute (split operands) 259 registers against 162 at D 32, 263 against 236 at
+// D 64, one wave per SIMD against three or two, which calls of many tiles lose
+// more by (see dkdv_launch).
+template <typename IO, int CT, int D, int NW, int KT, int KU, int QS, bool VEC, bool FS, bool HAT>
 __global__ void __launch_bounds__(NW * 64)
 bwd_dkdv_kernel(const BwdParams p) {
   using C = Comp<CT>;
@@ -771,7 +776,7 @@ bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool TR = sizeof(S) == 2;
   // two query blocks in flight per trip, where the registers allow it (at D 32
   // it measured +11%: the second block's accumulators cost a wave per SIMD)
-  constexpr bool PIPE2 = sizeof(S) == 2 && (KT == 1 || D == 64);
+  constexpr bool PIPE2 = sizeof(S) == 2 && KU == KT && (KT == 1 || D == 64);
 
   static_assert(!FS || CT == DT_BF16, "fp16 logit operands go with bf16 compute");
   __shared__ __attribute__((aligned(16))) S sQ[QS * LDQ];
@@ -1036,21 +1041,20 @@ bwd_dkdv_kernel(const BwdParams p) {
     lds_barrier();
     }
 
-    // S and dP of query block j for the wave's key subtiles; each Q-hat / dO
-    // fragment is read once and feeds all KT of them.  (Read again per subtile,
+    // S and dP of query block j for key subtiles u0 .. u0 + KU - 1; each Q-hat /
+    // dO fragment is read once and feeds all of them.  (Read again per subtile,
     // the LDS bound this kernel: D 64, N 4096, 48 planes, backward 804 -> 733
-    // us; fp32 compute, N 197, 16 planes 62 -> 55 us; bit-identical.)  -LSE2 and -delta of
-    // queries 32j + 8lg + e, e = 4h + i, seed the accumulators of half h
-    // (P = exp2(S), dP - delta need no arithmetic; queries >= N have
-    // -LSE2 = -inf, so P = 0).
-    using Acc = f32x4[KT][2];
-    auto sp = [&](int j, Acc& sacc, Acc& pacc) __attribute__((always_inline)) {
+    // us; bit-identical.)  -LSE2 and -delta of queries 32j + 8lg + e, e = 4h + i,
+    // seed the accumulators of half h (P = exp2(S), dP - delta need no
+    // arithmetic; queries >= N have -LSE2 = -inf, so P = 0).
+    using Acc = f32x4[KU][2];
+    auto sp = [&](int j, int u0, Acc& sacc, Acc& pacc) __attribute__((always_inline)) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const f32x4 nl2 = *reinterpret_cast<const f32x4*>(&sL2[32 * j + 8 * lg + 4 * h]);
         const f32x4 ndl = *reinterpret_cast<const f32x4*>(&sDl[32 * j + 8 * lg + 4 * h]);
 #pragma unroll
-        for (int u = 0; u < KT; ++u) {
+        for (int u = 0; u < KU; ++u) {
           sacc[u][h] = nl2;
           pacc[u][h] = ndl;
         }
@@ -1067,22 +1071,22 @@ bwd_dkdv_kernel(const BwdParams p) {
             a = C::lds(&sQ[ql * LDQ + 32 * s + 8 * lg]);
           const Frag b = C::lds(&sG[ql * LDQ + 32 * s + 8 * lg]);
 #pragma unroll
-          for (int u = 0; u < KT; ++u) {
-            sacc[u][h] = LC::mma(a, kf[u][s], sacc[u][h]);
-            pacc[u][h] = C::mma(b, vf[u][s], pacc[u][h]);
+          for (int u = 0; u < KU; ++u) {
+            sacc[u][h] = LC::mma(a, kf[u0 + u][s], sacc[u][h]);
+            pacc[u][h] = C::mma(b, vf[u0 + u][s], pacc[u][h]);
           }
         }
       }
     };
     // P and dS of query block j from its S / dP, then dV += P dO and
-    // dK-hat += dS Q-hat; each dO^T / Q-hat^T fragment feeds all KT subtiles.
-    auto pdk = [&](int j, const Acc& sacc, const Acc& pacc) __attribute__((always_inline)) {
+    // dK-hat += dS Q-hat; each dO^T / Q-hat^T fragment feeds all KU subtiles.
+    auto pdk = [&](int j, int u0, const Acc& sacc, const Acc& pacc) __attribute__((always_inline)) {
       // Keys >= N (lane key kv0 + lr; a whole subtile past it included) need
       // no mask: their K-hat and V rows are zero, and P and dS there only
       // reach the dK / dV rows of those keys, which are never stored.
-      Frag pf[KT], dsf[KT], dsfl[KT];
+      Frag pf[KU], dsf[KU], dsfl[KU];
 #pragma unroll
-      for (int u = 0; u < KT; ++u) {
+      for (int u = 0; u < KU; ++u) {
         float pv[8], dsv[8];
 #pragma unroll
         for (int h = 0; h < 2; ++h)
@@ -1114,32 +1118,42 @@ bwd_dkdv_kernel(const BwdParams p) {
           aq = C::lds(&sQt[(16 * d + lr) * LDT + 32 * j + 8 * lg]);
         }
 #pragma unroll
-        for (int u = 0; u < KT; ++u) {
-          dvacc[u][d] = C::mma(ag, pf[u], dvacc[u][d]);
-          if constexpr (FS) dkacc[u][d] = C::mma(aq, dsfl[u], dkacc[u][d]);
-          dkacc[u][d] = C::mma(aq, dsf[u], dkacc[u][d]);
+        for (int u = 0; u < KU; ++u) {
+          dvacc[u0 + u][d] = C::mma(ag, pf[u], dvacc[u0 + u][d]);
+          if constexpr (FS) dkacc[u0 + u][d] = C::mma(aq, dsfl[u], dkacc[u0 + u][d]);
+          dkacc[u0 + u][d] = C::mma(aq, dsf[u], dkacc[u0 + u][d]);
         }
       }
     };
 
-    if (kv_first < N) {   // wave-uniform
-      const int nbj = rows / 32;
+    const int nbj = rows / 32;
+    if constexpr (KU < KT) {
+      for (int j = 0; j < nbj; ++j) {
+#pragma unroll
+        for (int u0 = 0; u0 < KT; u0 += KU) {
+          if (kv_first + 16 * u0 >= N) continue;   // wave-uniform
+          Acc sacc, pacc;
+          sp(j, u0, sacc, pacc);
+          pdk(j, u0, sacc, pacc);
+        }
+      }
+    } else if (kv_first < N) {   // wave-uniform
       if constexpr (PIPE2) {
         // Two query blocks per trip: the S / dP products of block j+1 go to the
         // MFMA pipe before block j's probabilities are computed on the VALU (a
         // ragged last block recomputes block j instead and skips its update).
         for (int j = 0; j < nbj; j += 2) {
           Acc sA, pA, sB, pB;
-          sp(j, sA, pA);
-          sp(min(j + 1, nbj - 1), sB, pB);
-          pdk(j, sA, pA);
-          if (j + 1 < nbj) pdk(j + 1, sB, pB);
+          sp(j, 0, sA, pA);
+          sp(min(j + 1, nbj - 1), 0, sB, pB);
+          pdk(j, 0, sA, pA);
+          if (j + 1 < nbj) pdk(j + 1, 0, sB, pB);
         }
       } else {
         for (int j = 0; j < nbj; ++j) {
           Acc sacc, pacc;
-          sp(j, sacc, pacc);
-          pdk(j, sacc, pacc);
+          sp(j, 0, sacc, pacc);
+          pdk(j, 0, sacc, pacc);
         }
       }
     }
@@ -1355,22 +1369,36 @@ static hipError_t dkdv_launch(const BwdParams& p0, hipStream_t st) {
   constexpr bool FS = f16_logits(CT, D);
   BwdParams p = p0;
   const int grid = p.n_wg = p.B * p.H * p.n_blk;
+  // Shared fragment reads, except in fp32 compute for calls past 2 tiles per CU,
+  // or past 1 where a plane has one tile.  Measured (us, backward, one read per
+  // subtile / shared; tiles in brackets), D 32: N 324, 64 planes [192] 51 / 43;
+  // 128 of N 361 [384] 85 / 82; 192 of N 401 [768] 128 / 131; 1024 of N 324 [3072]
+  // 382 / 453; D 64: 64 of N 324 [192] 90 / 78; 128 of N 400 [512] 183 / 176;
+  // 192 of N 289 [576] 208 / 210; 96 of N 1025 [864] 451 / 437; 640 of N 289
+  // [1920] 543 / 590; one tile: N 65 [256] 35 / 32; [512] 63 / 67.
+  if constexpr (CT == DT_F32 && SH::KV_KT > 1) {
+    if (grid > kCus * (p.n_blk == 1 ? 1 : 2)) {
+      hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, 1, SH::KV_QS, false, FS, false>), dim3(grid),
+                         dim3(SH::KV_NW * 64), 0, st, p);
+      return hipGetLastError();
+    }
+  }
   // (fp32 compute has no registers to spare for the prefetch)
   if constexpr (CT != DT_F32) {
     if (p.vec_q && p.vec_do) {
       if constexpr (FS) {
         if (p.qhat_f) {
-          hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_QS, true, FS, true>),
+          hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_KT, SH::KV_QS, true, FS, true>),
                              dim3(grid), dim3(SH::KV_NW * 64), 0, st, p);
           return hipGetLastError();
         }
       }
-      hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_QS, true, FS, false>), dim3(grid),
+      hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_KT, SH::KV_QS, true, FS, false>), dim3(grid),
                          dim3(SH::KV_NW * 64), 0, st, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_QS, false, FS, false>), dim3(grid),
+  hipLaunchKernelGGL((bwd_dkdv_kernel<IO, CT, D, SH::KV_NW, SH::KV_KT, SH::KV_KT, SH::KV_QS, false, FS, false>), dim3(grid),
                      dim3(SH::KV_NW * 64), 0, st, p);
   return hipGetLastError();
 }

@@ -1354,8 +1354,6 @@ template <> struct FwdShape<128> { static constexpr int NW = 8, QT = 1, KC = 64,
 // 512 registers (VGPRs plus AGPRs): the O accumulators alone are 64 per wave.
 template <> struct FwdShape<256> { static constexpr int NW = 4, QT = 1, KC = 32, TABROWS = 0; };
 
-constexpr int kFwdCus = 256;   // CUs of the chip
-
 // Query subtiles per wave at D = 128: two with 16-bit tensors and 16-bit
 // compute, so that every staged K-hat chunk (rotated and converted once per
 // item) serves twice the queries; their Q rows
@@ -1380,7 +1378,7 @@ int fwd_block_rows(int D, int io, int ct) {
 // fp16 compute [96] 25.2 / 20.8, [384] 18.1 / 26.2.  Bit-identical (bf16).
 int fwd_call_rows(int D, int io, int ct, int planes, int N) {
   const int rows = fwd_block_rows(D, io, ct), one = FwdShape<128>::NW * 16;
-  if (D == 128 && rows > one && (int64_t)planes * ((N + one - 1) / one) <= kFwdCus) return one;
+  if (D == 128 && rows > one && (int64_t)planes * ((N + one - 1) / one) <= kCus) return one;
   return rows;
 }
 int fwd_threads(int D) {

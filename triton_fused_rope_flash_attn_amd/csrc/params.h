@@ -85,6 +85,7 @@ enum FwdVariant : int {
   FWD_SHORT = 3,    // short-plane kernel (short.hip)
 };
 
+constexpr int kCus = 256;   // CUs of the chip
 // Workgroups of 256 threads a launch may hold: HIP refuses 2^32 threads or more.
 constexpr int64_t kMaxWorkgroups = (int64_t(1) << 24) - 1;
 
