@@ -99,6 +99,19 @@ def _route(planes, N, D, io, ct, which):
     (16, 197, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
     (24, 1025, 128, _lib.BF16, _lib.BF16, (0, 128), (3, 128)),
     (384, 1025, 128, _lib.BF16, _lib.BF16, (0, 256), (3, 128)),
+    # head_dim 128 in fp16: 64-row tiles up to one per CU (12 x 785: 156 tiles), or up to two where
+    # the 128-row ones pass one (96 x 289: 480 and 288), and the 256-row items where they fill their
+    # rounds (128 x 325: 256 items, 192 x 257: 192, 512 x 441: 1024)
+    (12, 785, 128, _lib.F16, _lib.F16, (2, 64), (4, 64)),
+    (28, 785, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
+    (96, 289, 128, _lib.F16, _lib.F16, (2, 64), (4, 64)),
+    (128, 325, 128, _lib.F16, _lib.F16, (0, 256), (4, 64)),
+    (192, 257, 128, _lib.F16, _lib.F16, (0, 256), (1, 128)),
+    (160, 257, 128, _lib.F16, _lib.F16, (2, 128), (1, 128)),
+    (512, 441, 128, _lib.F16, _lib.F16, (0, 256), (4, 64)),
+    (224, 441, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
+    (256, 361, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
+    (64, 1025, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
 ])
 def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
     """which = 2 and 3: the kernels that a call takes."""
@@ -109,16 +122,16 @@ def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
 def test_routes_stay_within_the_launch_limit(lib):
     """A launch holds fewer than 2^32 threads: calls whose tiles need 2^24 workgroups
     of 256 keep the kernels that take any number of planes (the largest tensors
-    here are 4 GB)."""
+    of the short planes are 4 GB)."""
     m = 2 ** 24
     for io in (_lib.BF16, _lib.F32):
         assert _route(m - 1, 4, 32, io, io, 2)[0] == 3 and _route(m, 4, 32, io, io, 2)[0] == 0
         assert _route(m // 2 - 1, 4, 32, io, io, 3)[0] == 5 and _route(m // 2, 4, 32, io, io, 3)[0] == 1
-    # head_dim 128: the K-hat pass takes 17 blocks of 16 rows per two planes of 257 rows
-    n = 2 * (m - 1) // 17
+    # head_dim 128: the K-hat pass takes 65 blocks of 16 rows per two planes of 1025 rows
+    n = 2 * (m - 1) // 65
     for planes, streamed in ((n - 1, True), (n + 3, False)):
-        assert (_route(planes, 257, 128, _lib.F16, _lib.F16, 2)[0] == 2) == streamed
-        desc = _lib.make_desc(planes, 1, 257, 128, 256, True, _lib.F16, _lib.F16, 0.1)
+        assert (_route(planes, 1025, 128, _lib.F16, _lib.F16, 2)[0] == 2) == streamed
+        desc = _lib.make_desc(planes, 1, 1025, 128, 1024, True, _lib.F16, _lib.F16, 0.1)
         assert (_lib.fwd_workspace_elems(desc) != 0) == streamed
 
 

@@ -331,9 +331,28 @@ bool stream_shape(const farope_attn_desc* d) {
 // Measured (us, fwd_kernel / streamed, the K-hat pass included): D 64, N 577,
 // 384 planes 89 / 59; N 257, 1536 planes 90 / 78; N 256 52 / 59; N 170, 3072
 // planes 81 / 107.  D 32: N 257, 512 planes 32 / 25; N 256 15 / 20.  D 128, fp16: N
-// 257, 384 planes 54 / 47; N 577 137 / 120; N 1025, 12 planes 51 / 24; N 4096, 24
-// planes 295 / 207.
-bool fwd_stream(const farope_attn_desc* d) { return stream_shape(d) && d->seq_len > kPlaneMaxN; }
+// 257, 384 planes 54 / 47; N 577 137 / 117; N 1025, 12 planes 51 / 24; N 4096, 24
+// planes 297 / 205.
+//
+// At D 128 fwd_kernel's 256-row items, one per CU at a time, stay the better
+// ones where they fill their rounds (us, "planes x N [items]", fwd_kernel /
+// streamed): one round of at least 5/8 (6/8 where the last rows take a launch of
+// their own), planes up to 800 rows: 80 x 441 [160] 26 / 28.4, 64 x 529 [192] 31 /
+// 33.8, 128 x 325 [256] 24.1 / 27.9, 192 x 257 [192] 31 / 32.1, but 64 x 361 [128] 19 /
+// 18.1, 64 x 1025 [256] 66 / 62; more rounds, all full, planes up to 512 rows that
+// 128-row tiles would not pad less: 512 x 441 [1024] 94 / 105, 1024 x 257 [1024]
+// 104 / 118, but 224 x 441 [448] 49 / 48.5, 256 x 361 [512] 45 / 38.7, 256 x 1024
+// [1024] 178 / 180.
+bool fwd_stream(const farope_attn_desc* d) {
+  if (!stream_shape(d) || d->seq_len <= kPlaneMaxN) return false;
+  const int planes = d->batch * d->heads, N = d->seq_len;
+  const int64_t tiles = (int64_t)planes * cdiv(N, kStreamTileRows);
+  if (d->head_dim != 128 || tiles <= kCus || stream_rows(planes, N, 128, false) < kStreamTileRows) return true;
+  const int rows = fwd_block_rows(128, d->io_dtype, d->compute_dtype);
+  const int64_t items = (int64_t)planes * main_blocks(planes, N, rows), rounds = (items + kCus - 1) / kCus;
+  if (rounds == 1) return N > 800 || 8 * items < kCus * (tail_of(planes, N, rows) ? 6 : 5);
+  return N > 512 || 2 * items > tiles || 20 * items < 19 * rounds * kCus;
+}
 // Backward: planes past the one-pass kernel's 256 rows at head_dim 64, and past
 // the same length at 32 and 128.  (Not N = 257 at 64 and 128: its workspace of
 // delta rows alone is what callers of the C ABI allocate.)  Measured (us,

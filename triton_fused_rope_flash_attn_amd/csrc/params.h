@@ -151,9 +151,17 @@ constexpr int kStreamThreads = 256;
 // 44.3 / 39.8, [480] 23.7 / 23.8, [960] 36.4 / 37.6; D 32: [320] 54.7 / 44.2, [640]
 // 18.5 / 16.9.  Backward, D 64: [33] 51.6 / 37.1, [60] 31.0 / 22.7, [240] 34.2 / 31.4,
 // [384] 108 / 102, [480] 48.4 / 50.0, [960] 81 / 87; D 32: [320] 133 / 119, [640] 39.2 /
-// 38.6.  (The backward's results are the same bit for bit.)
+// 38.6.  (The backward's results are the same bit for bit.)  Forward at D 128,
+// where two workgroups of either size fit on a CU: 64-row tiles while they fit one
+// per CU, and where they fit two per CU and the 128-row tiles do not fit one
+// ("planes x N", 128 / 64 rows): 12 x 785 23.7 / 19.0, 28 x 785 26.3 / 27.6, 34 x 901
+// 41.3 / 33.9, 96 x 289 24.0 / 19.4, 64 x 785 39.4 / 48.5, 16 x 3137 99.8 / 138.
 inline int stream_rows(int planes, int N, int D, bool backward) {
   const int64_t tiles = (int64_t)planes * ((N + kStreamTileRows - 1) / kStreamTileRows);
+  if (D == 128 && !backward) {
+    const int64_t half = (int64_t)planes * ((N + kStreamTileRows / 2 - 1) / (kStreamTileRows / 2));
+    return half <= kCus || (half <= 2 * kCus && tiles > kCus) ? kStreamTileRows / 2 : kStreamTileRows;
+  }
   return tiles <= (D == 32 ? 768 : backward ? 400 : 512) ? kStreamTileRows / 2 : kStreamTileRows;
 }
 // K-hat * c2 rows [planes][N][D] of 16-bit K (any vector-access strides), in
