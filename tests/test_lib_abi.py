@@ -112,6 +112,15 @@ def _route(planes, N, D, io, ct, which):
     (224, 441, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
     (256, 361, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
     (64, 1025, 128, _lib.F16, _lib.F16, (2, 128), (4, 64)),
+    # fp32 compute at head_dim 64: planes of 65 to 112 rows in the 128-row tiles where these fill the chip
+    (256, 65, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (384, 65, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (512, 65, 64, _lib.F32, _lib.F32, (3, 64), (1, 128)),
+    (640, 82, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (1536, 101, 64, _lib.F32, _lib.F32, (3, 64), (1, 128)),
+    (1536, 122, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (1536, 64, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    (1536, 101, 32, _lib.F32, _lib.F32, (3, 64), (5, 64)),
 ])
 def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
     """which = 2 and 3: the kernels that a call takes."""
