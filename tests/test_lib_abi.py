@@ -121,6 +121,13 @@ def _route(planes, N, D, io, ct, which):
     (1536, 122, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
     (1536, 64, 64, _lib.F32, _lib.F32, (3, 64), (5, 64)),
     (1536, 101, 32, _lib.F32, _lib.F32, (3, 64), (5, 64)),
+    # fp32 tensors in 16-bit compute at head_dim 64, past 64 rows: up to 300 Ki rows
+    (2048, 122, 64, _lib.F32, _lib.BF16, (3, 64), (0, 256)),
+    (3072, 100, 64, _lib.F32, _lib.F16, (3, 64), (0, 256)),
+    (3072, 122, 64, _lib.F32, _lib.BF16, (0, 256), (0, 256)),
+    (8192, 64, 64, _lib.F32, _lib.BF16, (3, 64), (0, 256)),
+    (8192, 122, 32, _lib.F32, _lib.BF16, (3, 64), (1, 128)),
+    (8192, 122, 64, _lib.BF16, _lib.BF16, (3, 64), (0, 256)),
 ])
 def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
     """which = 2 and 3: the kernels that a call takes."""

@@ -391,21 +391,29 @@ bool short_shape(const farope_attn_desc* d, int per) {
   if (d->head_dim != 64 && d->head_dim != 32) return false;
   return d->seq_len <= kPlaneMaxN && short_tiles(d) * per <= kMaxWorkgroups;
 }
-// Forward: up to 128 rows always, longer planes while the call has too few of
-// them to fill the chip with one workgroup (fwd_kernel) or one wave
-// (fwd_plane) a plane, whose time hardly changes up to 256 or 1024 planes.
-// Measured (us, those kernels / short; "planes x N"): bf16 D 64: 3072 x 122
-// 58 / 42, 144 x 121 8.9 / 7.6; fwd_plane 12 x 197 22.6 / 7.2, 96 23.0 / 8.3,
-// 384 26.0 / 21.9, 576 27.4 / 31.9; fwd_kernel 120 x 144 10.5 / 7.9, 192 x 144
-// 10.7 / 11.5, 120 x 256 12.4 / 8.5, 384 x 256 22.3 / 23.0; fp32 compute 96 x
-// 197 26.6 / 18.8, 192 28.1 / 28.7.  D 32: 4096 x 64 42 / 14, 4096 x 144 76 / 61,
-// 512 x 197 14.3 / 14.0, 4096 x 197 84 / 87; fp32 compute 512 x 197 29.9 / 30.1,
-// 4096 x 144 162 / 168.
+// Forward: up to 128 rows always (past 64 rows at head_dim 64, fp32 tensors in
+// 16-bit compute while the call's tensors fit the last-level cache: then their
+// loads bound it, and the persistent kernel's prefetch hides them better),
+// longer planes while the call has too few of them to fill the chip with one
+// workgroup (fwd_kernel) or one wave (fwd_plane) a plane, whose time hardly
+// changes up to 256 or 1024 planes.  Measured (us, those kernels / short;
+// "planes x N"): bf16 D 64: 3072 x 122 58 / 42, 144 x 121 8.9 / 7.6, 16384 x 122
+// 291 / 277; fp32 tensors in bf16, D 64: 2048 x 122 54 / 45, 3072 x 100 74 / 73,
+// 4096 x 65 72 / 72, 3072 x 122 84 / 93, 6144 x 81 117 / 128, 12288 x 122 300 /
+// 349, 8192 x 64 116 / 113; D 32 12288 x 122 227 / 177.  fwd_plane 12 x 197 22.6 /
+// 7.2, 96 23.0 / 8.3, 384 26.0 / 21.9, 576 27.4 / 31.9; fwd_kernel 120 x 144 10.5 /
+// 7.9, 192 x 144 10.7 / 11.5, 120 x 256 12.4 / 8.5, 384 x 256 22.3 / 23.0; fp32
+// compute 96 x 197 26.6 / 18.8, 192 28.1 / 28.7.  D 32: 4096 x 64 42 / 14, 4096 x
+// 144 76 / 61, 512 x 197 14.3 / 14.0, 4096 x 197 84 / 87; fp32 compute 512 x 197
+// 29.9 / 30.1, 4096 x 144 162 / 168.
+constexpr int64_t kCacheRows = 300 * 1024;   // four fp32 tensors of 64 channels: 315 MB
 bool fwd_short(const farope_attn_desc* d) {
   if (!short_shape(d, 1)) return false;
-  if (d->seq_len <= 128) return true;
-  const int64_t t = short_tiles(d);
   const bool f32 = d->compute_dtype == FAROPE_F32;
+  if (d->seq_len <= 128)
+    return d->head_dim == 32 || d->seq_len <= kShortTileRows || f32 || d->io_dtype != FAROPE_F32 ||
+           (int64_t)d->batch * d->heads * d->seq_len <= kCacheRows;
+  const int64_t t = short_tiles(d);
   if (d->head_dim == 32) return f32 ? t <= 1024 : d->seq_len <= 192 || t <= 2048;
   return t <= (fwd_plane(d, true) ? 1536 : 512);
 }
