@@ -128,6 +128,10 @@ def _route(planes, N, D, io, ct, which):
     (8192, 64, 64, _lib.F32, _lib.BF16, (3, 64), (0, 256)),
     (8192, 122, 32, _lib.F32, _lib.BF16, (3, 64), (1, 128)),
     (8192, 122, 64, _lib.BF16, _lib.BF16, (3, 64), (0, 256)),
+    # 16-bit tensors at head_dim 64, 49 to 64 rows in the backward: likewise
+    (4096, 64, 64, _lib.BF16, _lib.BF16, (3, 64), (5, 64)),
+    (5120, 64, 64, _lib.F16, _lib.F16, (3, 64), (0, 256)),
+    (8192, 37, 64, _lib.BF16, _lib.BF16, (3, 64), (5, 64)),
 ])
 def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
     """which = 2 and 3: the kernels that a call takes."""

@@ -406,7 +406,8 @@ bool short_shape(const farope_attn_desc* d, int per) {
 // compute 96 x 197 26.6 / 18.8, 192 28.1 / 28.7.  D 32: 4096 x 64 42 / 14, 4096 x
 // 144 76 / 61, 512 x 197 14.3 / 14.0, 4096 x 197 84 / 87; fp32 compute 512 x 197
 // 29.9 / 30.1, 4096 x 144 162 / 168.
-constexpr int64_t kCacheRows = 300 * 1024;   // four fp32 tensors of 64 channels: 315 MB
+// (four fp32 or eight 16-bit tensors of 64 channels: 315 MB)
+constexpr int64_t kCacheRows = 300 * 1024;
 bool fwd_short(const farope_attn_desc* d) {
   if (!short_shape(d, 1)) return false;
   const bool f32 = d->compute_dtype == FAROPE_F32;
@@ -421,18 +422,20 @@ bool fwd_short(const farope_attn_desc* d) {
 // replaces two kernels of 128-row tiles), but for fp32 planes of 65 to 112 rows
 // at head_dim 64, which fill one 128-row tile better than two 64-row ones, in
 // calls that fill the chip with those tiles.  16-bit compute at head_dim 64: 33
-// to 64 rows in 16-bit tensors always; else against the one-pass kernel while two
-// workgroups a CU hold the whole call (with N <= 32 that kernel's delta is the
-// more exact one and stays); fp32 tensors likewise, at head_dim 32 up to 64
-// rows always.  Measured (us, those kernels / short): fp32 compute, D 64: 16 x
-// 197 54.7 / 15.6, 1536 x 197 731 / 607, 1536 x 64 151 / 53, 256 x 65 35.0 / 35.1,
-// 384 x 65 60 / 52, 448 x 101 75 / 67, 640 x 65 90 / 86, 512 x 65 63 / 69, 900 x
-// 65 115 / 122, 1536 x 65 169 / 200, 2048 x 81 239 / 279, 1024 x 100 140 / 148,
-// 1536 x 122 233 / 233; D 32 4096 x 144 682 / 350.  bf16 D 32: 4096 x 64 75 / 34,
-// 4096 x 197 270 / 257, 4096 x 256 303 / 302.  bf16 D 64: 3072 x 64 60.6 / 56.0, 12
-// x 197 16.9 / 9.2, 48 x 197 17.3 / 11.7, 96 x 197 17.6 / 17.6, 192 x 197 18.1 /
-// 29.0.  fp32 tensors in bf16: D 32 4096 x 64 97 / 67, 1024 x 197 82 / 97; D 64 48
-// x 197 26.0 / 17.9, 3072 x 64 91 / 113.
+// to 64 rows in 16-bit tensors always, past 48 rows while the call's tensors fit
+// the last-level cache; else against the one-pass kernel while two workgroups a
+// CU hold the whole call (with N <= 32 that kernel's delta is the more exact one
+// and stays); fp32 tensors likewise, at head_dim 32 up to 64 rows always.
+// Measured (us, those kernels / short): fp32 compute, D 64: 16 x 197 54.7 /
+// 15.6, 1536 x 197 731 / 607, 1536 x 64 151 / 53, 256 x 65 35.0 / 35.1, 384 x 65
+// 60 / 52, 448 x 101 75 / 67, 640 x 65 90 / 86, 512 x 65 63 / 69, 900 x 65 115 /
+// 122, 1536 x 65 169 / 200, 2048 x 81 239 / 279, 1024 x 100 140 / 148, 1536 x
+// 122 233 / 233; D 32 4096 x 144 682 / 350.  bf16 D 32: 4096 x 64 75 / 34, 4096
+// x 197 270 / 257, 4096 x 256 303 / 302.  bf16 D 64: 3072 x 64 60.6 / 56.0, 4096
+// x 64 80 / 75, 5120 x 64 107 / 111, 8192 x 64 166 / 181, 8192 x 49 156 / 154,
+// 8192 x 37 142 / 132, 12 x 197 16.9 / 9.2, 48 x 197 17.3 / 11.7, 96 x 197 17.6
+// / 17.6, 192 x 197 18.1 / 29.0.  fp32 tensors in bf16: D 32 4096 x 64 97 / 67,
+// 1024 x 197 82 / 97; D 64 48 x 197 26.0 / 17.9, 3072 x 64 91 / 113.
 bool bwd_short(const farope_attn_desc* d) {
   if (!short_shape(d, 2)) return false;
   if (d->compute_dtype == FAROPE_F32) {
@@ -443,7 +446,9 @@ bool bwd_short(const farope_attn_desc* d) {
   }
   const bool io16 = d->io_dtype != FAROPE_F32, one = d->seq_len <= kShortTileRows;
   if (d->head_dim == 64 && d->seq_len <= 32) return false;
-  if (d->head_dim == 32 ? io16 || one : io16 && one) return true;
+  if (d->head_dim == 32 && (io16 || one)) return true;
+  if (d->head_dim == 64 && io16 && one)
+    return d->seq_len <= 48 || (int64_t)d->batch * d->heads * d->seq_len <= kCacheRows;
   return 2 * short_tiles(d) <= 512;
 }
 
