@@ -132,6 +132,12 @@ def _route(planes, N, D, io, ct, which):
     (4096, 64, 64, _lib.BF16, _lib.BF16, (3, 64), (5, 64)),
     (5120, 64, 64, _lib.F16, _lib.F16, (3, 64), (0, 256)),
     (8192, 37, 64, _lib.BF16, _lib.BF16, (3, 64), (5, 64)),
+    # head_dim 128 in bf16: 128-row items up to one per CU, unless they leave 2 to 8 rows to the
+    # tail kernel that 256-row items take in (901 = 7 * 128 + 5 = 3 * 256 + 133)
+    (24, 900, 128, _lib.BF16, _lib.BF16, (0, 256), (2, 128)),
+    (24, 901, 128, _lib.BF16, _lib.BF16, (0, 256), (2, 128)),
+    (24, 785, 128, _lib.BF16, _lib.BF16, (0, 128), (3, 128)),
+    (8, 257, 128, _lib.BF16, _lib.BF16, (0, 128), (3, 128)),
 ])
 def test_call_routes(lib, planes, N, D, io, ct, fwd, bwd):
     """which = 2 and 3: the kernels that a call takes."""

@@ -1372,14 +1372,16 @@ int fwd_block_rows(int D, int io, int ct) {
 }
 // Query rows per item of a call: at D = 128 one subtile per wave (128 rows)
 // while those items still fit the chip at one workgroup per CU; two subtiles
-// (256 rows) halve the staging per query once every CU is busy.  Measured (us,
-// 256 / 128 rows; 128-row items in brackets): bf16 [24] 20.4 / 15.2, [108] 58.5 /
-// 45.0, [192] 21.5 / 16.3, [240] 36.8 / 27.1, [432] 60.4 / 79.9, [768] 326 / 348;
-// fp16 compute [96] 25.2 / 20.8, [384] 18.1 / 26.2.  Bit-identical (bf16).
+// (256 rows) halve the staging per query once every CU is busy, and stay where
+// 128-row items would leave rows to the tail kernel that they take in (N = 901).
+// Measured (us, 256 / 128 rows; 128-row items in brackets): bf16 [24] 20.4 / 15.2,
+// [108] 58.5 / 45.0, [192] 21.5 / 16.3, [240] 36.8 / 27.1, [432] 60.4 / 79.9, [768]
+// 326 / 348; 24 planes of N 901 46.6 / 52.0, 16 of N 1157 54.5 / 61.7; fp16 compute
+// [96] 25.2 / 20.8, [384] 18.1 / 26.2.  Bit-identical (bf16).
 int fwd_call_rows(int D, int io, int ct, int planes, int N) {
   const int rows = fwd_block_rows(D, io, ct), one = FwdShape<128>::NW * 16;
-  if (D == 128 && rows > one && (int64_t)planes * ((N + one - 1) / one) <= kCus) return one;
-  return rows;
+  if (D != 128 || rows <= one || (int64_t)planes * ((N + one - 1) / one) > kCus) return rows;
+  return tail_rows(N, one) > 1 && !tail_rows(N, rows) ? rows : one;
 }
 int fwd_threads(int D) {
   return 64 * (D == 32    ? FwdShape<32>::NW
