@@ -382,6 +382,40 @@ def test_fp32_split_backward_of_many_tiles(side, has_cls, D, B, H):
     _compare(f"many-fp32-tiles-N{N}-D{D}", [t[:2] for t in many], ref, tol_max=1e-4, tol_mean=1e-5)
 
 
+# calls past the limits of the short-plane and streamed kernels, which the smaller
+# batches of the other tests take: (side, has_cls, D, io, planes, forward and
+# backward variant)
+@pytest.mark.parametrize("side,has_cls,D,io,planes,fwd,bwd", [
+    (12, True, 64, "bf16", 400, 0, 0), (13, True, 64, "fp16", 400, 0, 0), (14, False, 64, "bf16", 400, 1, 0),
+    (14, True, 64, "fp16", 400, 1, 0), (15, True, 64, "bf16", 400, 0, 0), (16, False, 64, "fp16", 400, 0, 0),
+    (8, False, 64, "bf16", 5120, 3, 0), (9, True, 64, "bf16", 400, 3, 0), (5, False, 64, "bf16", 400, 3, 0),
+    (11, True, 64, "amp", 2560, 0, 0), (12, True, 64, "amp", 400, 0, 0),
+    (15, False, 32, "bf16", 540, 0, 5), (14, True, 32, "fp16", 540, 0, 5), (14, True, 32, "amp", 540, 0, 1),
+    (14, True, 32, "fp32", 300, 0, 5), (12, True, 64, "fp32", 200, 0, 5),
+    (8, True, 64, "fp32", 512, 3, 1), (10, True, 64, "fp32", 1040, 3, 1),
+    (18, True, 128, "fp16", 128, 0, 4), (16, True, 128, "fp16", 192, 0, 1), (30, True, 128, "bf16", 4, 0, 2),
+])
+def test_calls_past_the_short_and_streamed_kernels(side, has_cls, D, io, planes, fwd, bwd):
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16}.get(io, torch.float32)
+    N = side * side + int(has_cls)
+    ct = _lib.BF16 if io == "amp" else _lib.DTYPE_CODE[dt]
+    desc = _lib.make_desc(planes // 4, 4, N, D, side * side, has_cls, _lib.DTYPE_CODE[dt], ct, D ** -0.5)
+    assert (_lib.tile_config(desc, 2)[0], _lib.tile_config(desc, 3)[0]) == (fwd, bwd)
+    _say(f"case {planes} planes of N={N} D={D} {io}")
+    g = torch.Generator(device=DEV).manual_seed(12)
+    q, k, v, do = (torch.randn(planes // 4, 4, N, D, generator=g, device=DEV).to(dt) for _ in range(4))
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    ours = _run_ours(q, k, v, do, table, has_cls, autocast_dtype=torch.bfloat16 if io == "amp" else None)
+    ref = _ref(q, k, v, do, table, has_cls)
+    tag = f"past-{planes}x{N}-D{D}-{io}"
+    if io == "fp32":
+        _compare(tag, ours, ref, tol_max=1e-4, tol_mean=1e-5)
+    else:
+        # (fp32 tensors in bf16: the mean's bound as for the short planes, four operands off by 2^-9
+        # of entries of mean size 0.3)
+        _compare(tag, ours, ref, out_dtype=torch.bfloat16 if io == "amp" else dt, tol_mean=2e-3 if io == "amp" else TOL_MEAN)
+
+
 def test_stride0_dout_from_sum():
     cfg = dict(CONFIGS["vit_b"], B=4)
     q, k, v, _ = make_inputs(cfg, DEV)

@@ -61,8 +61,9 @@ def test_streamed_tiles(side, has_cls, D, dt, B, H):
     if B > 2 and N > 600:
         pytest.skip("the 128-row tiles' remainders are covered by the shorter planes")
     code = {"bf16": _lib.BF16, "fp16": _lib.F16}[dt]
-    rows = _lib.tile_config(_lib.make_desc(B, H, N, D, N - int(has_cls), has_cls, code, code, 0.1), 1)[1]
-    assert rows == (64 if B == 2 or D == 128 else 128)
+    desc = _lib.make_desc(B, H, N, D, N - int(has_cls), has_cls, code, code, 0.1)
+    assert _lib.tile_config(desc, 2)[:2] == (2, 64 if B == 2 else 128)
+    assert _lib.tile_config(desc, 3)[:2] == (4, 64 if B == 2 or D == 128 else 128)
     dt = {"bf16": torch.bfloat16, "fp16": torch.float16}[dt]
     print(f"streamed N={N} D={D} {dt}", flush=True)
     table = CosSinTable(ROPE_BASE, side, D, device=DEV)

@@ -3,7 +3,7 @@ farope_attn_bwd (caller workspace), both called through the C ABI.
 
 Workspace-path calls in a row (N = 257 at D = 128 through the stored-dS
 backward, N = 257 at D = 64 through the split path, then a smaller D = 128
-problem) and one one-pass call: the same kernels run with their workspace in
+problem), one one-pass call and one of the short-plane kernels: the same kernels run with their workspace in
 the library's static array instead of a caller buffer, so dQ, dK and dV must
 be identical bit for bit.  The second call reuses the array the first one left behind.
 The one-pass backward uses no workspace at all, so the no-alloc entry also
@@ -47,7 +47,7 @@ def _one(B, H, side, has_cls, D, seed):
     for name, a, b in zip(("dQ", "dK", "dV"), got, ref):
         assert torch.isfinite(a).all(), name
         assert torch.equal(a, b), f"{name}: max diff {(a.float() - b.float()).abs().max().item():.3e}"
-    return _lib.tile_config(desc, 1)[0]
+    return _lib.tile_config(desc, 3)[0]   # the kernels the calls took
 
 
 def test_noalloc_one_pass_beyond_static_rows():
@@ -66,7 +66,7 @@ def test_noalloc_one_pass_beyond_static_rows():
     scale = 1.0 / math.sqrt(D)
     o, lse, res = torch.ops.farope.attn_fwd(q, k, v, rope, N - 1, True, scale, _lib.BF16)
     desc = _lib.make_desc(B, H, N, D, N - 1, True, _lib.BF16, _lib.BF16, scale)
-    assert _lib.tile_config(desc, 1)[0] == 0 and _lib.bwd_workspace_elems(desc) == 0
+    assert _lib.tile_config(desc, 3)[0] == 0 and _lib.bwd_workspace_elems(desc) == 0
     ref = [torch.empty_like(q) for _ in range(3)]
     _lib.attn_bwd(desc, q, k, v, o, do, lse, rope, *ref, None, res)
     got = [torch.full_like(q, float("nan")) for _ in range(3)]
@@ -84,4 +84,5 @@ def test_noalloc_matches_workspace_entry_two_calls():
     assert _one(2, 3, 16, True, 128, seed=24) == 3
     assert _one(4, 6, 16, True, 64, seed=21) == 1    # split path, N = 257
     assert _one(2, 3, 7, True, 128, seed=22) == 3    # smaller, stored-dS path (one ragged key tile)
-    assert _one(2, 4, 14, True, 64, seed=23) == 0    # one-pass path (no workspace used)
+    assert _one(9, 12, 14, True, 64, seed=23) == 0   # one-pass path (no workspace used)
+    assert _one(2, 4, 14, True, 64, seed=25) == 5    # short-plane kernels (none either)
