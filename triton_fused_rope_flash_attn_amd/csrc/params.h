@@ -151,18 +151,24 @@ constexpr int kStreamThreads = 256;
 // 44.3 / 39.8, [480] 23.7 / 23.8, [960] 36.4 / 37.6; D 32: [320] 54.7 / 44.2, [640]
 // 18.5 / 16.9.  Backward, D 64: [33] 51.6 / 37.1, [60] 31.0 / 22.7, [240] 34.2 / 31.4,
 // [384] 108 / 102, [480] 48.4 / 50.0, [960] 81 / 87; D 32: [320] 133 / 119, [640] 39.2 /
-// 38.6.  (The backward's results are the same bit for bit.)  Forward at D 128,
-// where two workgroups of either size fit on a CU: 64-row tiles while they fit one
-// per CU, and where they fit two per CU and the 128-row tiles do not fit one
-// ("planes x N", 128 / 64 rows): 12 x 785 23.7 / 19.0, 28 x 785 26.3 / 27.6, 34 x 901
-// 41.3 / 33.9, 96 x 289 24.0 / 19.4, 64 x 785 39.4 / 48.5, 16 x 3137 99.8 / 138.
+// 38.6.  (The backward's results are the same bit for bit.)
+//
+// At D 128 two workgroups of either size fit on a CU.  Forward: 64-row tiles
+// while they fit one per CU, and where they fit two per CU and the 128-row tiles
+// do not fit one ("planes x N", 128 / 64 rows): 12 x 785 23.7 / 19.0, 28 x 785 26.3 /
+// 27.6, 34 x 901 41.3 / 33.9, 96 x 289 24.0 / 19.4, 64 x 785 39.4 / 48.5, 16 x 3137
+// 99.8 / 138.  Backward, whose dQ tiles alone take it: 64 rows up to 400 tiles of
+// 128, past 1024 rows while either size fits as above: 40 x 785 95 / 90, 48 x 901
+// 122 / 121; 24 x 1157 94 / 92, 24 x 1297 111 / 102, 24 x 2025 235 / 254, 16 x 3136 358
+// / 406.
 inline int stream_rows(int planes, int N, int D, bool backward) {
   const int64_t tiles = (int64_t)planes * ((N + kStreamTileRows - 1) / kStreamTileRows);
-  if (D == 128 && !backward) {
-    const int64_t half = (int64_t)planes * ((N + kStreamTileRows / 2 - 1) / (kStreamTileRows / 2));
-    return half <= kCus || (half <= 2 * kCus && tiles > kCus) ? kStreamTileRows / 2 : kStreamTileRows;
+  bool half = tiles <= (D == 32 ? 768 : backward ? 400 : 512);
+  if (D == 128 && (!backward || N > 1024)) {
+    const int64_t h = (int64_t)planes * ((N + kStreamTileRows / 2 - 1) / (kStreamTileRows / 2));
+    half = backward ? tiles <= kCus || h <= 2 * kCus : h <= kCus || (h <= 2 * kCus && tiles > kCus);
   }
-  return tiles <= (D == 32 ? 768 : backward ? 400 : 512) ? kStreamTileRows / 2 : kStreamTileRows;
+  return half ? kStreamTileRows / 2 : kStreamTileRows;
 }
 // K-hat * c2 rows [planes][N][D] of 16-bit K (any vector-access strides), in
 // the compute type: what both passes stream.
@@ -180,7 +186,7 @@ inline int64_t khat_blocks(int64_t planes, int N, int D) {
   return (int64_t)((N + rows - 1) / rows) * ((planes + kKhatPlanes - 1) / kKhatPlanes);
 }
 hipError_t launch_stream_khat(const KhatParams& p, int ct, int D, hipStream_t st);
-// Forward over 128-query tiles; khat from launch_stream_khat.
+// Forward over 128- or 64-query tiles; khat from launch_stream_khat.
 hipError_t launch_fwd_stream(const FwdParams& p, const void* khat, int io, int D, hipStream_t st);
 hipError_t launch_bwd_stream(const BwdParams& p, int io, int D, hipStream_t st);
 
