@@ -154,10 +154,11 @@ int farope_attn_fwd(const farope_attn_desc* desc,
 /*
  * farope_attn_fwd with a caller workspace of farope_attn_fwd_workspace_elems(desc)
  * fp32 elements (16-byte aligned; NULL: as farope_attn_fwd).  Where that is not
- * 0 (16-bit tensors computed in their own type, head_dim 32 or 64, or 128 in
- * fp16, and seq_len > 256) and every tensor allows vector access, the rotated
- * K rows are written there once and streamed by every query tile; otherwise it
- * is not used.  No counterpart in the reference.
+ * 0 (16-bit tensors computed in their own type and seq_len > 256, head_dim 32 or
+ * 64, or 128 in fp16 but for calls whose 256-row items fill the chip) and every
+ * tensor allows vector access, the rotated K rows are written there once and
+ * streamed by every query tile; otherwise it is not used.  No counterpart in the
+ * reference.
  */
 size_t farope_attn_fwd_workspace_elems(const farope_attn_desc* desc);
 int farope_attn_fwd_ws(const farope_attn_desc* desc,

@@ -354,12 +354,14 @@ bool fwd_stream(const farope_attn_desc* d) {
   return N > 512 || 2 * items > tiles || 20 * items < 19 * rounds * kCus;
 }
 // Backward: planes past the one-pass kernel's 256 rows at head_dim 64, and past
-// the same length at 32 and 128.  (Not N = 257 at 64 and 128: its workspace of
-// delta rows alone is what callers of the C ABI allocate.)  Measured (us,
-// bwd_dq_kernel + bwd_dkdv_kernel / streamed): D 64, N 577, 384 planes 264 /
-// 159; N 4096, 48 planes 795 / 597; N 324, 24 planes 42 / 24.  D 32, N 257, 512
-// planes 71 / 43.  D 128, fp16: N 577, 384 planes 497 / 368; N 1024 1024 / 888; N 1025, 12 planes 142 / 58; N 289, 96
-// planes 69 / 42.
+// the same length at 32 and 128.  Not N = 257 at 64 and 128, though streaming is
+// the faster one there too (D 64, 12 planes 48.8 / 14.5, 384 98 / 62, 1536 295 /
+// 226; D 128, 384 161 / 122): its workspace is held to the delta rows alone, a
+// size that tests/test_lib_abi.py fixes.  Measured (us, bwd_dq_kernel +
+// bwd_dkdv_kernel / streamed): D 64, N 577, 384 planes 264 / 159; N 4096, 48
+// planes 795 / 597; N 324, 24 planes 42 / 24.  D 32, N 257, 512 planes 71 / 43.
+// D 128, fp16: N 577, 384 planes 497 / 368; N 1024 1024 / 888; N 1025, 12 planes
+// 142 / 58; N 289, 96 planes 69 / 42.
 bool bwd_stream(const farope_attn_desc* d) {
   return stream_shape(d) && d->seq_len > kPlaneMaxN + (d->head_dim >= 64 ? 1 : 0);
 }

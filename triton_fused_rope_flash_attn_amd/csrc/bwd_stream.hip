@@ -14,8 +14,9 @@
 // The rows that a tile streams (K-hat and V, or Q-hat and dO) are then ready
 // to use, so they go from memory straight to LDS (16 bytes per lane, no
 // staging registers, no VALU) in stages of 64 rows, double-buffered with one
-// barrier per stage.  Workgroups are 4 waves of 32 rows each, two (dK/dV) or
-// three (dQ) on a CU: their barriers are independent, so one workgroup's
+// barrier per stage.  Workgroups are 4 waves of 32 rows each (16 in 64-row tiles,
+// which dK/dV always takes at head_dim 128), two on a CU, or three (dQ at
+// head_dim 32 and 64): their barriers are independent, so one workgroup's
 // MFMAs run under another's softmax and stage waits.
 //
 // Bound by instruction issue (MFMA and the softmax VALU; every operand crosses

@@ -8,14 +8,14 @@
 // stream_khat_kernel writes the rotated, scaled K rows once; the tiles then
 // stream K-hat and V from memory straight to LDS (16 bytes per lane, no
 // staging registers or VALU), in double-buffered stages of 64 keys with one
-// barrier each.  Three 4-wave workgroups run on a CU, so one's MFMAs fill the
-// time of another's softmax.
+// barrier each.  Three 4-wave workgroups run on a CU (two at head_dim 128, whose
+// stages take 64 KB), so one's MFMAs fill the time of another's softmax.
 //
 // Bound by the softmax VALU (16 exponentials, maxima and row-sum adds per lane
 // and 32 x 32 block against 16 MFMAs).  Measured against fwd_kernel (one 8-wave
 // workgroup per CU, 256-row tiles; us): D 64, N 577, 384 planes 89 -> 58 (K-hat
 // pass 11); N 4096, 48 planes 285 -> 207; N 1025, 64 planes 46 -> 37; D 32, N
-// 3970, 10 planes 81 -> 43; D 128, fp16, N 577, 384 planes 137 -> 118.  Two or
+// 3970, 10 planes 81 -> 43; D 128, fp16, N 577, 384 planes 137 -> 117.  Two or
 // four workgroups per CU (D 32 and 64): within 1%.
 #include <type_traits>
 

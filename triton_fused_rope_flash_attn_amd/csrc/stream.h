@@ -7,7 +7,7 @@
 
 namespace farope {
 
-constexpr int kStreamNW = 4;                  // waves per workgroup, 32 rows each
+constexpr int kStreamNW = 4;                  // waves per workgroup, 32 rows each (16 in 64-row tiles)
 static_assert(32 * kStreamNW == kStreamTileRows && 64 * kStreamNW == kStreamThreads, "");
 constexpr int kStageRows = 64;                // streamed rows per stage
 

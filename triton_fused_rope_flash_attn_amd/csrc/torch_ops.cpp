@@ -8,7 +8,7 @@
 // autograd node whose backward runs on the engine's thread without taking the
 // interpreter lock.  Small calls are bound by exactly that host work: a
 // training pass of 96 planes of 197 rows took 226 us around 43 us of kernels
-// with the Python kernels, 63 us with these.
+// with the Python kernels, 70 to 75 us with these (box to box).
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
