@@ -416,6 +416,41 @@ def test_calls_past_the_short_and_streamed_kernels(side, has_cls, D, io, planes,
         _compare(tag, ours, ref, out_dtype=torch.bfloat16 if io == "amp" else dt, tol_mean=2e-3 if io == "amp" else TOL_MEAN)
 
 
+# (D, io, side, has_cls, planes): the one-pass kernel (its delta from P and dP too, N = 4),
+# the split kernels at every head_dim, the short, streamed and stored-dS ones
+@pytest.mark.parametrize("D,io,side,has_cls,planes", [
+    (64, "bf16", 2, False, 2), (64, "fp16", 14, True, 100), (64, "amp", 14, True, 100), (64, "bf16", 16, True, 2),
+    (64, "amp", 17, False, 2), (32, "amp", 14, True, 100), (128, "fp16", 14, True, 2), (128, "amp", 6, True, 2),
+    (256, "bf16", 6, True, 2), (256, "fp16", 15, False, 2),
+    (64, "bf16", 6, True, 2), (64, "bf16", 17, False, 2), (128, "bf16", 15, False, 2), (64, "fp32", 17, False, 2),
+])
+@pytest.mark.parametrize("which", ["k", "v"])
+@pytest.mark.parametrize("stride", [0, 16])
+def test_overlapping_key_and_value_rows(D, io, side, has_cls, planes, which, stride):
+    """K or V with one row stride for all rows: 0 (one row for every token) or less
+    than D (rows overlap).  Rows past the plane's end then read real values, which
+    must not reach dQ."""
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16}.get(io, torch.float32)
+    N = side * side + int(has_cls)
+    _say(f"case overlapping {which} rows, stride {stride}: {planes} planes of N={N} D={D} {io}")
+    g = torch.Generator(device=DEV).manual_seed(13)
+    t = {c: torch.randn(planes, 1, N, D, generator=g, device=DEV).to(dt) for c in ("q", "k", "v", "do")}
+    base = torch.randn(planes, 1, (N - 1) * stride + D, generator=g, device=DEV).to(dt)
+    t[which] = base.as_strided((planes, 1, N, D), (*base.stride()[:2], stride, 1))
+    leaves = [t[c].detach().requires_grad_() for c in "qkv"]
+    table = CosSinTable(ROPE_BASE, side, D, device=DEV)
+    with torch.autocast("cuda", torch.bfloat16, enabled=io == "amp"):
+        o = sdpa_triton_fa_rope(*leaves, table, H_img=side, has_cls=has_cls)
+    ours = (o.detach(), *torch.autograd.grad(o, leaves, t["do"]))
+    ref = _ref(*(t[c].float().contiguous() for c in ("q", "k", "v", "do")), table, has_cls)
+    tag = f"overlap-{which}{stride}-N{N}-D{D}-{io}"
+    if io == "fp32":
+        _compare(tag, ours, ref, tol_max=1e-4, tol_mean=1e-5)
+    else:
+        # (fp32 tensors in bf16: the mean's bound as for the short planes)
+        _compare(tag, ours, ref, out_dtype=torch.bfloat16 if io == "amp" else dt, tol_mean=2e-3 if io == "amp" else TOL_MEAN)
+
+
 def test_stride0_dout_from_sum():
     cfg = dict(CONFIGS["vit_b"], B=4)
     q, k, v, _ = make_inputs(cfg, DEV)

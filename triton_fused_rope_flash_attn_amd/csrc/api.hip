@@ -111,7 +111,8 @@ int vec_ok(const void* p, const int64_t s[4], int es, int n_rows, int head_dim) 
 
 // Written tensors additionally need rows that do not overlap (row stride >=
 // head_dim): the kernels then store rows >= N unconditionally and rely on
-// the descriptor range to drop them.
+// the descriptor range to drop them.  So do K and V of the one-pass and split
+// backward, whose dQ counts on keys >= N having zero rows.
 int vec_out_ok(const void* p, const int64_t s[4], int es, int n_rows, int head_dim) {
   return vec_ok(p, s, es, n_rows, head_dim) && s[2] >= head_dim;
 }
@@ -527,8 +528,8 @@ int bwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
   copy4(p.sdo, dout_stride); copy4(p.sdq, dq_stride); copy4(p.sdk, dk_stride);
   copy4(p.sdv, dv_stride);
   p.vec_q = vec_ok(q, q_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_k = vec_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_v = vec_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_k = vec_out_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_v = vec_out_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
   p.vec_o = vec_ok(o, o_stride, es, desc->seq_len, desc->head_dim);
   p.vec_do = vec_ok(dout, dout_stride, es, desc->seq_len, desc->head_dim);
   p.vec_dq = vec_out_ok(dq, dq_stride, es, desc->seq_len, desc->head_dim);
@@ -536,20 +537,21 @@ int bwd_impl(const farope_attn_desc* desc, const void* q, const int64_t q_stride
   p.vec_dv = vec_out_ok(dv, dv_stride, es, desc->seq_len, desc->head_dim);
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int D = desc->head_dim;
-  if (bwd_short(desc) && p.vec_q && p.vec_k && p.vec_v && p.vec_o && p.vec_do && p.vec_dq && p.vec_dk && p.vec_dv)
-    return launch_rc(launch_bwd_short(p, desc->io_dtype, desc->compute_dtype, D, st));
+  // vector access to every tensor, with rows of K and V that may overlap: the
+  // short, streamed and stored-dS kernels make keys >= N zero rows themselves
+  const bool vec = p.vec_q && vec_ok(k, k_stride, es, desc->seq_len, D) && vec_ok(v, v_stride, es, desc->seq_len, D) &&
+                   p.vec_o && p.vec_do && p.vec_dq && p.vec_dk && p.vec_dv;
+  if (bwd_short(desc) && vec) return launch_rc(launch_bwd_short(p, desc->io_dtype, desc->compute_dtype, D, st));
   if (fused) {
     p.n_blk = 1;
     return launch_rc(launch_bwd_fused(p, desc->io_dtype, desc->compute_dtype, st));
   }
   // the stored-dS backward (the static workspace only when all of it fits)
-  if (ds_possible(desc) && p.vec_q && p.vec_k && p.vec_v && p.vec_o && p.vec_do && p.vec_dq &&
-      p.vec_dk && p.vec_dv && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
+  if (ds_possible(desc) && vec && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
       (!static_ws || ds_ws(desc).total <= kScratchFloats))
     return ds_pass(p, desc, delta_ws, st);
   // streamed tiles (the static workspace only when all of it fits)
-  if (bwd_stream(desc) && p.vec_q && p.vec_k && p.vec_v && p.vec_o && p.vec_do && p.vec_dq &&
-      p.vec_dk && p.vec_dv && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
+  if (bwd_stream(desc) && vec && reinterpret_cast<uintptr_t>(delta_ws) % 16 == 0 &&
       (!static_ws || stream_ws(desc).total <= kScratchFloats)) {
     const StreamWs w = stream_ws(desc);
     p.row_stat = delta_ws + w.nl;
@@ -832,8 +834,8 @@ int farope_attn_bwd_dq(const farope_attn_desc* desc, const void* q, const int64_
   copy4(p.sq, q_stride); copy4(p.sk, k_stride); copy4(p.sv, v_stride);
   copy4(p.sdo, dout_stride); copy4(p.sdq, dq_stride);
   p.vec_q = vec_ok(q, q_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_k = vec_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
-  p.vec_v = vec_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_k = vec_out_ok(k, k_stride, es, desc->seq_len, desc->head_dim);
+  p.vec_v = vec_out_ok(v, v_stride, es, desc->seq_len, desc->head_dim);
   p.vec_do = vec_ok(dout, dout_stride, es, desc->seq_len, desc->head_dim);
   p.vec_dq = vec_out_ok(dq, dq_stride, es, desc->seq_len, desc->head_dim);
   return dq_pass(p, desc, false, static_cast<hipStream_t>(stream));
